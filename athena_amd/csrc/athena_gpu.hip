@@ -800,6 +800,16 @@ __global__ void __launch_bounds__(WG) k_flux_div(MeshK M, const double *__restri
   }
 }
 
+// Element at byte offset o of a wavefront-uniform base: scalar base, 32-bit lane offset
+// (o made opaque in the block of its use, or the compiler widens it once for all uses and
+// forms every address with 64-bit vector adds).
+__device__ __forceinline__ double ldb(const double *base, unsigned o) {
+  return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + o);
+}
+__device__ __forceinline__ void stb(double *base, unsigned o, double v) {
+  *reinterpret_cast<double *>(reinterpret_cast<char *>(base) + o) = v;
+}
+
 //========================================================================================
 // Kernel 2: corner EMFs, Field::ComputeCornerE 3-D branch (calculate_corner_e.cpp:129-230)
 // One thread per edge position (k,j,i) in [ks..ke+1]x[js..je+1]x[is..ie+1]; the
@@ -916,13 +926,19 @@ __device__ __forceinline__ void corner_body(const MeshK &M, const CornerArgs &ca
 }
 
 // Z-marching corner EMFs (tile option with tx < 0, tz = planes per segment): a
-// work-group owns a TI x TJ tile of (i, j) edge positions (TI = the box width up to 256,
-// TJ = 256 / (TI+1) - 1 rows but at least one, so that for TI < 255 its 256 threads
-// stage the (TI+1) x (TJ+1) cells in one pass) and walks up a segment of planes.  The cell-centred E of the
-// (TI+1) x (TJ+1) cells of a plane that the tile's edges touch is evaluated once into
-// LDS (planes k-1 and k, double-buffered), and every thread carries the four face values
-// of plane k-1 that its edges need from the previous step, so each array element is
-// read from memory about once instead of once per neighbouring work-group.
+// work-group owns a TI x TJ tile of (i, j) edge positions (TI = the box width up to 255,
+// TJ = 256 / (TI+1) - 1 rows but at least one, so that its 256 threads hold the
+// (TI+1) x (TJ+1) cells the edges touch) and walks up a segment of planes.  Thread t holds
+// the cell at its place in that rectangle: it loads the cell's velocity and field and the
+// face EMFs and weights of the three faces on its low sides, each once per plane, a plane
+// ahead of their use; the values of the cells one row down and one column left come through
+// LDS (two buffers, one barrier per plane), those of the plane below are kept in registers.
+//
+// Bound by the vector caches (their lines wait on L2 for 80 % of the launch) and by the
+// partly written lines at the row ends (10 % in a bare copy of the same pattern).  Every
+// value loaded per edge that needs it, between two barriers a plane, in segments of 8
+// planes, took 132 us over 64 blocks of 32^3 cells, 772 us over 64 of 64^3, 27 us over 64
+// of 16^3; each loaded once, 118, 698 and 17 us.
 struct MarchGeom {
   int ti, tj, nti, ntj, ks, nks;
 };
@@ -931,19 +947,59 @@ __host__ __device__ __forceinline__ MarchGeom march_geom(const MeshK &M, int ks)
   int lo[3], n[3];
   kind_box(M, KK_CORNER, lo, n);
   MarchGeom G;
-  G.ti = (n[0] < WG) ? n[0] : WG;
-  G.tj = WG / (G.ti + 1) - 1;   // stage (ti+1) x (tj+1) cells in one pass
-  if (G.tj < 1) G.tj = 1;
-  if (G.tj > n[1]) G.tj = n[1];
+  G.ti = (n[0] < WG) ? n[0] : WG - 1;
+  if (G.ti > WG / 2 - 1) {   // at least one row of edges: equal tiles of at most 127 columns
+    const int m = (n[0] + WG / 2 - 2) / (WG / 2 - 1);
+    G.ti = (n[0] + m - 1) / m;
+  }
+  G.tj = WG / (G.ti + 1) - 1;
   G.nti = (n[0] + G.ti - 1) / G.ti;
   G.ntj = (n[1] + G.tj - 1) / G.tj;
-  G.ks = ks;
+  G.tj = (n[1] + G.ntj - 1) / G.ntj;   // equal tiles
   G.nks = (n[2] + ks - 1) / ks;
+  G.ks = (n[2] + G.nks - 1) / G.nks;   // tallest segment
   return G;
 }
 
+// Values a thread passes to its neighbours per plane: 7 face values and 3 cell-centred E.
+constexpr int MARCH_LDS_VALUES = 10;
+
 __host__ __device__ __forceinline__ int march_lds_doubles(const MarchGeom &G) {
-  return 2 * 3 * (G.ti + 1) * (G.tj + 1);
+  return 2 * MARCH_LDS_VALUES * (G.ti + 1) * (G.tj + 1);
+}
+
+// What a thread holds of one plane: the weights and EMFs of its cell's low faces, and the
+// cell's velocity and field.
+struct MarchPlane {
+  double w1, w2, w3, e2x1, e3x1, e1x2, e3x2, e1x3, e2x3, vx, vy, vz, b1, b2, b3;
+};
+
+__device__ __forceinline__ MarchPlane march_load(const MeshK &M, const CornerArgs &ca, int g,
+                                                 int k, unsigned oc, unsigned o1) {
+  asm volatile("" : "+v"(oc), "+v"(o1));
+  const long n = M.ncell, pc = static_cast<long>(M.nc2) * M.nc1;
+  const long q1 = static_cast<long>(g) * M.nf1 + k * (static_cast<long>(M.nc2) * (M.nc1 + 1));
+  const long q2 = static_cast<long>(g) * M.nf2 + k * (static_cast<long>(M.nc2 + 1) * M.nc1);
+  const long q3 = static_cast<long>(g) * M.nf3 + k * pc;
+  const double *w = ca.w + static_cast<long>(g) * NHYDRO * n + k * pc;
+  const double *b = ca.bcc + static_cast<long>(g) * 3 * n + k * pc;
+  MarchPlane P;
+  P.w1 = ldb(ca.wx1 + q1, o1);
+  P.e2x1 = ldb(ca.e2x1 + q1, o1);
+  P.e3x1 = ldb(ca.e3x1 + q1, o1);
+  P.w2 = ldb(ca.wx2 + q2, oc);
+  P.e1x2 = ldb(ca.e1x2 + q2, oc);
+  P.e3x2 = ldb(ca.e3x2 + q2, oc);
+  P.w3 = ldb(ca.wx3 + q3, oc);
+  P.e1x3 = ldb(ca.e1x3 + q3, oc);
+  P.e2x3 = ldb(ca.e2x3 + q3, oc);
+  P.vx = ldb(w + IVX * n, oc);
+  P.vy = ldb(w + IVY * n, oc);
+  P.vz = ldb(w + IVZ * n, oc);
+  P.b1 = ldb(b + IB1 * n, oc);
+  P.b2 = ldb(b + IB2 * n, oc);
+  P.b3 = ldb(b + IB3 * n, oc);
+  return P;
 }
 
 template <bool SR>
@@ -959,85 +1015,98 @@ __device__ __forceinline__ void corner_march(const MeshK &M, const CornerArgs &c
   const int seg = r % G.nks;
   r /= G.nks;
   const int tjx = r % G.ntj, tix = r / G.ntj;
-  const int i0 = lo[0] + tix * G.ti, j0 = lo[1] + tjx * G.tj;
-  const int k0 = lo[2] + seg * G.ks;
-  const int k1 = (k0 + G.ks < lo[2] + n[2]) ? k0 + G.ks : lo[2] + n[2];
+  const int k0 = lo[2] + (seg * n[2]) / G.nks, k1 = lo[2] + ((seg + 1) * n[2]) / G.nks;
   const int iend = lo[0] + n[0] - 1, jend = lo[1] + n[1] - 1;   // last edge positions
   const int t = threadIdx.x;
-  const int i = i0 + t % G.ti, j = j0 + t / G.ti;
-  const bool act = (t / G.ti) < G.tj && i <= iend && j <= jend;
-  const int sw = G.ti + 1, ncs = sw * (G.tj + 1);   // staged cells i0-1.., j0-1.. per plane
-  const double *wb = ca.w + static_cast<long>(g) * NHYDRO * M.ncell;
-  const double *bb = ca.bcc + static_cast<long>(g) * 3 * M.ncell;
-  const long o1 = static_cast<long>(g) * M.nf1, o2 = static_cast<long>(g) * M.nf2;
-  const long o3 = static_cast<long>(g) * M.nf3;
-  auto stage = [&](double *dst, int kk) {
-    for (int c = t; c < ncs; c += WG) {
-      const int ci = i0 - 1 + c % sw, cj = j0 - 1 + c / sw;
-      if (ci > iend || cj > jend) continue;      // beyond the box: never read
-      const long q = cidx(M, kk, cj, ci);
-      dst[c] = cc_e<SR>(M, wb, bb, 0, q);
-      dst[ncs + c] = cc_e<SR>(M, wb, bb, 1, q);
-      dst[2 * ncs + c] = cc_e<SR>(M, wb, bb, 2, q);
+  const int sw = G.ti + 1, ncs = sw * (G.tj + 1);   // cells i0-1.., j0-1.. of a plane
+  const int rj = t / sw, ri = t - rj * sw;
+  const int i = lo[0] + tix * G.ti - 1 + ri, j = lo[1] + tjx * G.tj - 1 + rj;
+  const bool live = t < ncs && i <= iend && j <= jend;
+  const bool act = live && ri > 0 && rj > 0;
+  const unsigned oc = 8u * static_cast<unsigned>(j * M.nc1 + i);
+  const unsigned o1 = 8u * static_cast<unsigned>(j * (M.nc1 + 1) + i);
+  MarchPlane C{}, N{};
+  if (live) C = march_load(M, ca, g, k0 - 1, oc, o1);
+  // plane k-1: own face values, cell-centred E1 of this cell and one row down, E2 of this
+  // cell and one column left
+  double w1p = 0.0, w2p = 0.0, e12p = 0.0, e21p = 0.0, c0p = 0.0, c0jp = 0.0, c1p = 0.0;
+  double c1ip = 0.0;
+#pragma unroll 1
+  for (int k = k0 - 1; k < k1; ++k) {
+    double cc0 = C.vz * C.b2 - C.vy * C.b3;
+    double cc1 = C.vx * C.b3 - C.vz * C.b1;
+    double cc2 = C.vy * C.b1 - C.vx * C.b2;
+    if (SR) {
+      const double u0 = sqrt(1.0 + sq(C.vx) + sq(C.vy) + sq(C.vz));
+      cc0 = cc0 / u0;
+      cc1 = cc1 / u0;
+      cc2 = cc2 / u0;
     }
-  };
-  // face values of plane k-1 at (j, i): W1F, W2F, E1X2, E2X1
-  double w1p = 0.0, w2p = 0.0, e12p = 0.0, e21p = 0.0;
-  if (act) {
-    w1p = ca.wx1[o1 + f1idx(M, k0 - 1, j, i)];
-    w2p = ca.wx2[o2 + f2idx(M, k0 - 1, j, i)];
-    e12p = ca.e1x2[o2 + f2idx(M, k0 - 1, j, i)];
-    e21p = ca.e2x1[o1 + f1idx(M, k0 - 1, j, i)];
-  }
-  stage(lds_cc, k0 - 1);
-  int cur = 1;
-  for (int kq = k0; kq < k1; ++kq) {
-    const int k = __builtin_amdgcn_readfirstlane(kq);   // the same for the whole work-group
-    double *C = lds_cc + cur * 3 * ncs;
-    const double *P = lds_cc + (cur ^ 1) * 3 * ncs;
-    stage(C, k);
+    double *S = lds_cc + (k & 1) * (MARCH_LDS_VALUES * ncs);
+    if (live) {
+      S[t] = C.w1;
+      S[ncs + t] = C.w2;
+      S[2 * ncs + t] = C.w3;
+      S[3 * ncs + t] = C.e1x3;
+      S[4 * ncs + t] = C.e2x3;
+      S[5 * ncs + t] = C.e3x2;
+      S[6 * ncs + t] = C.e3x1;
+      S[7 * ncs + t] = cc0;
+      S[8 * ncs + t] = cc1;
+      S[9 * ncs + t] = cc2;
+      if (k + 1 < k1) N = march_load(M, ca, g, k + 1, oc, o1);
+    }
     __syncthreads();
     if (act) {
-      const double w1c = ca.wx1[o1 + f1idx(M, k, j, i)];
-      const double w2c = ca.wx2[o2 + f2idx(M, k, j, i)];
-      const double e12c = ca.e1x2[o2 + f2idx(M, k, j, i)];
-      const double e21c = ca.e2x1[o1 + f1idx(M, k, j, i)];
-      auto carried = [&](const double *a, long o, int comp, double prev, double curv) {
-        return [=, &M](int kk, int jj, int ii) {
-          if (kk < k) return prev;
-          if (jj == j && ii == i) return curv;
-          const long x = (comp == 0) ? f1idx(M, kk, jj, ii)
-                                     : ((comp == 1) ? f2idx(M, kk, jj, ii) : f3idx(M, kk, jj, ii));
-          return a[o + x];
+      const int dn = t - sw, lf = t - 1;         // one row down, one column left
+      const double cc0j = S[7 * ncs + dn], cc1i = S[8 * ncs + lf];
+      if (k >= k0) {
+        const double w1j = S[dn], w2i = S[ncs + lf], w3j = S[2 * ncs + dn];
+        const double w3i = S[2 * ncs + lf], e13j = S[3 * ncs + dn], e23i = S[4 * ncs + lf];
+        const double e32i = S[5 * ncs + lf], e31j = S[6 * ncs + dn];
+        const double cc2j = S[9 * ncs + dn], cc2i = S[9 * ncs + lf], cc2d = S[9 * ncs + dn - 1];
+        const double w1 = C.w1, w2 = C.w2, w3 = C.w3, e21 = C.e2x1, e31 = C.e3x1;
+        const double e12 = C.e1x2, e32 = C.e3x2, e13 = C.e1x3, e23 = C.e2x3;
+        auto sel = [](bool c, double x, double y) { return c ? x : y; };
+        auto W1F = [=](int kk, int jj, int) { return sel(kk < k, w1p, sel(jj < j, w1j, w1)); };
+        auto W2F = [=](int kk, int, int ii) { return sel(kk < k, w2p, sel(ii < i, w2i, w2)); };
+        auto W3F = [=](int, int jj, int ii) { return sel(jj < j, w3j, sel(ii < i, w3i, w3)); };
+        auto E2X1 = [=](int kk, int, int) { return sel(kk < k, e21p, e21); };
+        auto E3X1 = [=](int, int jj, int) { return sel(jj < j, e31j, e31); };
+        auto E1X2 = [=](int kk, int, int) { return sel(kk < k, e12p, e12); };
+        auto E3X2 = [=](int, int, int ii) { return sel(ii < i, e32i, e32); };
+        auto E1X3 = [=](int, int jj, int) { return sel(jj < j, e13j, e13); };
+        auto E2X3 = [=](int, int, int ii) { return sel(ii < i, e23i, e23); };
+        auto CC = [=](int comp, int kk, int jj, int ii) {
+          if (comp == 0) return sel(kk < k, sel(jj < j, c0jp, c0p), sel(jj < j, cc0j, cc0));
+          if (comp == 1) return sel(kk < k, sel(ii < i, c1ip, c1p), sel(ii < i, cc1i, cc1));
+          return sel(jj < j, sel(ii < i, cc2d, cc2j), sel(ii < i, cc2i, cc2));
         };
-      };
-      auto plain = [&](const double *a, long o, int comp) {
-        return [=, &M](int kk, int jj, int ii) {
-          const long x = (comp == 0) ? f1idx(M, kk, jj, ii)
-                                     : ((comp == 1) ? f2idx(M, kk, jj, ii) : f3idx(M, kk, jj, ii));
-          return a[o + x];
+        auto out = [&](int comp, double v) {
+          unsigned c = oc, f = o1;
+          asm volatile("" : "+v"(c), "+v"(f));
+          if (comp == 0)
+            stb(ca.e1 + static_cast<long>(g) * M.ne1 + k * (static_cast<long>(M.nc2 + 1) * M.nc1),
+                c, v);
+          else if (comp == 1)
+            stb(ca.e2 + static_cast<long>(g) * M.ne2 + k * (static_cast<long>(M.nc2) * (M.nc1 + 1)),
+                f, v);
+          else
+            stb(ca.e3 + static_cast<long>(g) * M.ne3 +
+                    k * (static_cast<long>(M.nc2 + 1) * (M.nc1 + 1)), f, v);
         };
-      };
-      auto cc = [&](int comp, int kk, int jj, int ii) {
-        const double *B = (kk < k) ? P : C;
-        return B[comp * ncs + (jj - j0 + 1) * sw + (ii - i0 + 1)];
-      };
-      auto out = [&](int comp, double v) {
-        if (comp == 0) ca.e1[static_cast<long>(g) * M.ne1 + e1idx(M, k, j, i)] = v;
-        else if (comp == 1) ca.e2[static_cast<long>(g) * M.ne2 + e2idx(M, k, j, i)] = v;
-        else ca.e3[static_cast<long>(g) * M.ne3 + e3idx(M, k, j, i)] = v;
-      };
-      corner_edges(k, j, i, carried(ca.wx1, o1, 0, w1p, w1c), carried(ca.wx2, o2, 1, w2p, w2c),
-                   plain(ca.wx3, o3, 2), carried(ca.e2x1, o1, 0, e21p, e21c),
-                   plain(ca.e3x1, o1, 0), carried(ca.e1x2, o2, 1, e12p, e12c),
-                   plain(ca.e3x2, o2, 1), plain(ca.e1x3, o3, 2), plain(ca.e2x3, o3, 2), cc, out);
-      w1p = w1c;
-      w2p = w2c;
-      e12p = e12c;
-      e21p = e21c;
+        corner_edges(k, j, i, W1F, W2F, W3F, E2X1, E3X1, E1X2, E3X2, E1X3, E2X3, CC, out);
+      }
+      c0jp = cc0j;
+      c1ip = cc1i;
     }
-    __syncthreads();
-    cur ^= 1;
+    w1p = C.w1;
+    w2p = C.w2;
+    e12p = C.e1x2;
+    e21p = C.e2x1;
+    c0p = cc0;
+    c1p = cc1;
+    C = N;
   }
 }
 
@@ -1850,6 +1919,7 @@ __global__ void __launch_bounds__(WG) k_corner_march_ens(const EnsMember *__rest
     const int2 mw = ens_item(map, v);
     const EnsMember &e = E[mw.x];
     corner_march<SR>(e.M, e.ca, mw.y, e.nwg[1], e.tile[1].tz);
+    __syncthreads();   // before the next item writes the LDS planes
   }
 }
 
@@ -2556,8 +2626,8 @@ long kind_chunks(const MeshK &M, int kind, TileK T) {
 }
 
 // Tile shapes the autotuner chooses from (index 0: linear chunks); indices 6 and 7 are
-// the z-march over segments of 8 and 16 planes: the corner kernel's (k_corner_march) and,
-// on single meshes, the flux kernel's (k_flux_zm).
+// the z-march: the corner kernel's (k_corner_march, segments of at most 2 and 4 planes) and,
+// on single meshes, the flux kernel's (k_flux_zm, segments of 8 and 16 planes).
 constexpr int NTILES = 8;
 constexpr TileK TILES[NTILES] = {{0, 0, 0}, {64, 4, 1}, {32, 8, 1}, {16, 16, 1}, {16, 4, 4},
                                  {8, 8, 4}, {-1, 0, 8}, {-1, 0, 16}};
@@ -2565,6 +2635,21 @@ constexpr TileK TILES[NTILES] = {{0, 0, 0}, {64, 4, 1}, {32, 8, 1}, {16, 16, 1},
 bool tile_ok(int kind, int t) { return TILES[t].tx >= 0 || kind == KK_CORNER; }
 // A single mesh also runs the flux kernel's z-march (k_flux_zm); ensembles do not.
 bool mesh_tile_ok(int kind, int t) { return tile_ok(kind, t) || kind == KK_FLUX; }
+
+// The z-march tile of a corner launch: segments of 2 planes (tile option 6) or 4 (7), one
+// where that would leave the GPU's 256 CUs short of three work-groups each.  Low segments
+// reload a plane more often but sweep memory nearly in order: segments of 1, 2, 3, 4, 8 and
+// 33 planes take 809, 699, 754, 755, 782 and 831 us over 64 blocks of 64^3 cells, 122, 118,
+// 122, 121, 123 and 122 us over 64 of 32^3.  One mesh of 8 blocks of 16^3: 7.0 us with
+// single planes, 8.3 with two.  share: this mesh's part of the launch (1 by itself).
+TileK corner_tile(const MeshK &M, TileK T, double share) {
+  if (T.tx >= 0) return T;
+  const MarchGeom G = march_geom(M, T.tz);
+  const double planes = static_cast<double>(G.nti) * G.ntj * (M.nx3 + 1) * M.nblocks;
+  const int h = static_cast<int>(planes / (3.0 * 256.0 * share) + 0.5);
+  T.tz = std::max(1, std::min(T.tz / 4, h));
+  return T;
+}
 
 // Dynamic LDS bytes of a corner launch with tile T.
 size_t corner_lds(const MeshK &M, TileK T) {
@@ -2722,9 +2807,9 @@ int launch_flux_dirs(ath_mesh *m, int order) {
 
 int launch_corner_args(ath_mesh *m, const CornerArgs &ca) {
   const MeshK &M = m->M;
-  const dim3 grid = kind_grid(m, KK_CORNER);
+  const TileK T = corner_tile(M, m->tile[KK_CORNER], 1.0);
+  const dim3 grid(static_cast<unsigned>(kind_chunks(M, KK_CORNER, T) * M.nblocks));
   ProfScope ps(m, KID_CORNER);
-  const TileK T = m->tile[KK_CORNER];
   const size_t lds = corner_lds(M, T);
   if (T.tx < 0 && m->d.relativistic)
     hipLaunchKernelGGL((k_corner_march<true>), grid, dim3(WG), lds, m->stream, M, ca, T);
@@ -3094,6 +3179,11 @@ int ens_build(ath_ensemble *e) {
   const int n = static_cast<int>(e->mem.size());
   std::vector<EnsMember> tab[2];
   std::vector<int2> map[KK_N], mapg;
+  auto cells_of = [](const ath_mesh *m) {
+    return static_cast<double>(m->M.nx1) * m->M.nx2 * m->M.nx3 * m->M.nblocks;
+  };
+  double cells = 0.0;
+  for (const auto *m : e->mem) cells += cells_of(m);
   for (int q = 0; q < n; ++q) {
     ath_mesh *m = e->mem[q];
     Regs r = regs_of(m);
@@ -3112,6 +3202,7 @@ int ens_build(ath_ensemble *e) {
       em.clk = m->clk;
       for (int k = 0; k < KK_N; ++k) {
         em.tile[k] = TILES[e->tile_idx[k]];
+        if (k == KK_CORNER) em.tile[k] = corner_tile(m->M, em.tile[k], cells_of(m) / cells);
         em.nwg[k] = static_cast<int>(kind_chunks(m->M, k, em.tile[k]) * m->M.nblocks);
       }
       if (em.nwg[KK_C2P] > m->ndtpart) return fail("dt partial buffer too small");
