@@ -11,15 +11,18 @@
 // synchronisation.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <cstdlib>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <limits>
 #include <map>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/athena_gpu.h"
@@ -55,6 +58,13 @@ namespace {
 
 constexpr int WG = 256;
 
+// Layout of the per-face outputs along one direction (fluxes, face EMFs, CT weights) within
+// one block: element (k, j, i) at k * plane + j * row + i - org, n doubles per component.
+struct FaceLayout {
+  int row, plane;
+  long org, n;
+};
+
 // Geometry and constants shared by all kernels of one mesh (passed by value).
 struct MeshK {
   int nx1, nx2, nx3, ng;
@@ -64,6 +74,8 @@ struct MeshK {
   long ncell;                 // nc1*nc2*nc3
   long nf1, nf2, nf3;         // x1f, x2f, x3f face-array sizes per block
   long ne1, ne2, ne3;         // x1e, x2e, x3e edge-array sizes per block
+  FaceLayout fl[3];           // per-face outputs of direction d
+  int packed;                 // 1: packed layout, the same for the three (pack_faces)
   int cstride;                // doubles of coordinate table per block
   int coff[3];                // offset of direction d inside the table
   const int *nbr;             // [nblocks][27] same-level neighbour gid, -1 across an
@@ -101,6 +113,11 @@ __device__ __forceinline__ long f2idx(const MeshK &M, int k, int j, int i) {
 }
 __device__ __forceinline__ long f3idx(const MeshK &M, int k, int j, int i) {
   return static_cast<long>(k) * (M.nc2 * M.nc1) + (j * M.nc1 + i);
+}
+template <int DIR>
+__device__ __forceinline__ long foidx(const MeshK &M, int k, int j, int i) {
+  const FaceLayout &L = M.fl[DIR];
+  return static_cast<long>(k) * L.plane + (j * L.row + i) - L.org;
 }
 // edge arrays: x1e (nc3+1, nc2+1, nc1), x2e (nc3+1, nc2, nc1+1), x3e (nc3, nc2+1, nc1+1)
 __device__ __forceinline__ long e1idx(const MeshK &M, int k, int j, int i) {
@@ -400,11 +417,21 @@ __device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, 
   fx[ivz] = f[IVZ];
   fx[IEN] = f[IEN];
   if (emit) {
-    o.ey[static_cast<long>(g) * nf + fi] = -f[IBY];
-    o.ez[static_cast<long>(g) * nf + fi] = f[IBZ];
+    const long q = static_cast<long>(g) * M.fl[DIR].n + foidx<DIR>(M, k, j, i);
+    o.ey[q] = -f[IBY];
+    o.ez[q] = f[IBZ];
     const double dxw = ct[fc];
-    o.wct[static_cast<long>(g) * nf + fi] = ct_weight(f[IDN], wl[IDN], wr[IDN], dxw, dt);
+    o.wct[q] = ct_weight(f[IDN], wl[IDN], wr[IDN], dxw, dt);
   }
+}
+
+template <int DIR>
+__device__ __forceinline__ void store_flux(const MeshK &M, int g, int k, int j, int i,
+                                           const FaceOut &o, const double *fx) {
+  const long nf = M.fl[DIR].n;
+  double *fb = o.flx + static_cast<long>(g) * NHYDRO * nf + foidx<DIR>(M, k, j, i);
+#pragma unroll
+  for (int n = 0; n < NHYDRO; ++n) fb[n * nf] = fx[n];
 }
 
 // face_flux with the fluxes written to Hydro::flux[DIR] (o.flx) as well.
@@ -415,14 +442,7 @@ __device__ __forceinline__ void flux_face(const MeshK &M, int g, int k, int j, i
                                           double dt) {
   double fx[NHYDRO];
   face_flux<DIR, ORDER, RS>(M, g, k, j, i, wb, bb, o, dt, true, fx);
-  long fi;
-  if (DIR == 0) fi = f1idx(M, k, j, i);
-  else if (DIR == 1) fi = f2idx(M, k, j, i);
-  else fi = f3idx(M, k, j, i);
-  const long nf = (DIR == 0) ? M.nf1 : ((DIR == 1) ? M.nf2 : M.nf3);
-  double *fb = o.flx + static_cast<long>(g) * NHYDRO * nf;
-#pragma unroll
-  for (int n = 0; n < NHYDRO; ++n) fb[n * nf + fi] = fx[n];
+  store_flux<DIR>(M, g, k, j, i, o, fx);
 }
 
 template <int DIR, int ORDER, int RS>
@@ -458,7 +478,16 @@ __device__ __forceinline__ void flux3_body(const MeshK &M, const double *__restr
   if (!map_kind(M, KK_FLUX, lw, nwg, T, g, i, j, k)) return;
   const double *wb = w + static_cast<long>(g) * NHYDRO * M.ncell;
   const double *bb = bcc + static_cast<long>(g) * 3 * M.ncell;
-  if (i >= M.is) flux_face<0, ORDER, RS>(M, g, k, j, i, wb, bb, o1, dt);
+  if (i >= M.is) {
+    flux_face<0, ORDER, RS>(M, g, k, j, i, wb, bb, o1, dt);
+  } else if (M.packed) {   // the row's unused first entry: complete its cache line
+    const long q = static_cast<long>(g) * M.fl[0].n + foidx<0>(M, k, j, i);
+    const double zero[NHYDRO] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    o1.ey[q] = 0.0;
+    o1.ez[q] = 0.0;
+    o1.wct[q] = 0.0;
+    store_flux<0>(M, g, k, j, i, o1, zero);
+  }
   if (j >= M.js) flux_face<1, ORDER, RS>(M, g, k, j, i, wb, bb, o2, dt);
   if (k >= M.ks) flux_face<2, ORDER, RS>(M, g, k, j, i, wb, bb, o3, dt);
 }
@@ -610,10 +639,7 @@ __global__ void __launch_bounds__(WG) k_flux_zm(MeshK M, const double *__restric
     for (int v = 0; v < NWAVE; ++v) wl[v] = __shfl_up(wl[v], 1, 64);
     if (live && i >= M.is) {
       face_solve<0, ORDER, RS>(M, g, k, j, i, wl, wr, o1, dt, true, fx);
-      const long fi = f1idx(M, k, j, i);
-      double *fb = o1.flx + static_cast<long>(g) * NHYDRO * M.nf1;
-#pragma unroll
-      for (int n = 0; n < NHYDRO; ++n) fb[n * M.nf1 + fi] = fx[n];
+      store_flux<0>(M, g, k, j, i, o1, fx);
     }
     // x2: both cells (indices made opaque again, so that the x1 addresses are not kept
     // alive through the x1 solve for reuse here)
@@ -625,10 +651,7 @@ __global__ void __launch_bounds__(WG) k_flux_zm(MeshK M, const double *__restric
       recon_cell<1, ORDER>(M, g, k, j - 1, i, wb, bb, t, wl);
       recon_cell<1, ORDER>(M, g, k, j, i, wb, bb, wr, t);
       face_solve<1, ORDER, RS>(M, g, k, j, i, wl, wr, o2, dt, true, fx);
-      const long fi = f2idx(M, k, j, i);
-      double *fb = o2.flx + static_cast<long>(g) * NHYDRO * M.nf2;
-#pragma unroll
-      for (int n = 0; n < NHYDRO; ++n) fb[n * M.nf2 + fi] = fx[n];
+      store_flux<1>(M, g, k, j, i, o2, fx);
     }
     // x3: low states of this cell, high states of the cell below carried in p3
     asm volatile("" : "+v"(k), "+v"(g), "+v"(j), "+v"(i));
@@ -637,10 +660,7 @@ __global__ void __launch_bounds__(WG) k_flux_zm(MeshK M, const double *__restric
     recon_cell<2, ORDER>(M, g, k, j, i, wb, bb, wr, wl);
     if (live && k >= M.ks) {
       face_solve<2, ORDER, RS>(M, g, k, j, i, p3, wr, o3, dt, true, fx);
-      const long fi = f3idx(M, k, j, i);
-      double *fb = o3.flx + static_cast<long>(g) * NHYDRO * M.nf3;
-#pragma unroll
-      for (int n = 0; n < NHYDRO; ++n) fb[n * M.nf3 + fi] = fx[n];
+      store_flux<2>(M, g, k, j, i, o3, fx);
     }
 #pragma unroll
     for (int v = 0; v < NWAVE; ++v) p3[v] = wl[v];
@@ -897,23 +917,22 @@ __device__ __forceinline__ void corner_body(const MeshK &M, const CornerArgs &ca
   const double *__restrict__ bcc = ca.bcc;
   const double *wb = w + static_cast<long>(g) * NHYDRO * M.ncell;
   const double *bb = bcc + static_cast<long>(g) * 3 * M.ncell;
-  const long o1 = static_cast<long>(g) * M.nf1, o2 = static_cast<long>(g) * M.nf2;
-  const long o3 = static_cast<long>(g) * M.nf3;
+  const long o1 = g * M.fl[0].n, o2 = g * M.fl[1].n, o3 = g * M.fl[2].n;
   const double *__restrict__ wx1 = ca.wx1 + o1, *__restrict__ wx2 = ca.wx2 + o2;
   const double *__restrict__ wx3 = ca.wx3 + o3;
   const double *__restrict__ e2x1 = ca.e2x1 + o1, *__restrict__ e3x1 = ca.e3x1 + o1;
   const double *__restrict__ e1x2 = ca.e1x2 + o2, *__restrict__ e3x2 = ca.e3x2 + o2;
   const double *__restrict__ e1x3 = ca.e1x3 + o3, *__restrict__ e2x3 = ca.e2x3 + o3;
   double *__restrict__ e1 = ca.e1, *__restrict__ e2 = ca.e2, *__restrict__ e3 = ca.e3;
-  auto W1F = [&](int kk, int jj, int ii) { return wx1[f1idx(M, kk, jj, ii)]; };
-  auto W2F = [&](int kk, int jj, int ii) { return wx2[f2idx(M, kk, jj, ii)]; };
-  auto W3F = [&](int kk, int jj, int ii) { return wx3[f3idx(M, kk, jj, ii)]; };
-  auto E2X1 = [&](int kk, int jj, int ii) { return e2x1[f1idx(M, kk, jj, ii)]; };
-  auto E3X1 = [&](int kk, int jj, int ii) { return e3x1[f1idx(M, kk, jj, ii)]; };
-  auto E1X2 = [&](int kk, int jj, int ii) { return e1x2[f2idx(M, kk, jj, ii)]; };
-  auto E3X2 = [&](int kk, int jj, int ii) { return e3x2[f2idx(M, kk, jj, ii)]; };
-  auto E1X3 = [&](int kk, int jj, int ii) { return e1x3[f3idx(M, kk, jj, ii)]; };
-  auto E2X3 = [&](int kk, int jj, int ii) { return e2x3[f3idx(M, kk, jj, ii)]; };
+  auto W1F = [&](int kk, int jj, int ii) { return wx1[foidx<0>(M, kk, jj, ii)]; };
+  auto W2F = [&](int kk, int jj, int ii) { return wx2[foidx<1>(M, kk, jj, ii)]; };
+  auto W3F = [&](int kk, int jj, int ii) { return wx3[foidx<2>(M, kk, jj, ii)]; };
+  auto E2X1 = [&](int kk, int jj, int ii) { return e2x1[foidx<0>(M, kk, jj, ii)]; };
+  auto E3X1 = [&](int kk, int jj, int ii) { return e3x1[foidx<0>(M, kk, jj, ii)]; };
+  auto E1X2 = [&](int kk, int jj, int ii) { return e1x2[foidx<1>(M, kk, jj, ii)]; };
+  auto E3X2 = [&](int kk, int jj, int ii) { return e3x2[foidx<1>(M, kk, jj, ii)]; };
+  auto E1X3 = [&](int kk, int jj, int ii) { return e1x3[foidx<2>(M, kk, jj, ii)]; };
+  auto E2X3 = [&](int kk, int jj, int ii) { return e2x3[foidx<2>(M, kk, jj, ii)]; };
   auto cc = [&](int comp, int kk, int jj, int ii) {
     return cc_e<SR>(M, wb, bb, comp, cidx(M, kk, jj, ii));
   };
@@ -975,24 +994,25 @@ struct MarchPlane {
 };
 
 __device__ __forceinline__ MarchPlane march_load(const MeshK &M, const CornerArgs &ca, int g,
-                                                 int k, unsigned oc, unsigned o1) {
-  asm volatile("" : "+v"(oc), "+v"(o1));
+                                                 int k, unsigned oc, unsigned o1, unsigned o2) {
+  asm volatile("" : "+v"(oc), "+v"(o1), "+v"(o2));
   const long n = M.ncell, pc = static_cast<long>(M.nc2) * M.nc1;
-  const long q1 = static_cast<long>(g) * M.nf1 + k * (static_cast<long>(M.nc2) * (M.nc1 + 1));
-  const long q2 = static_cast<long>(g) * M.nf2 + k * (static_cast<long>(M.nc2 + 1) * M.nc1);
-  const long q3 = static_cast<long>(g) * M.nf3 + k * pc;
+  // rows of x2 and x3 faces have the same pitch in either layout
+  const long q1 = g * M.fl[0].n + static_cast<long>(k) * M.fl[0].plane - M.fl[0].org;
+  const long q2 = g * M.fl[1].n + static_cast<long>(k) * M.fl[1].plane - M.fl[1].org;
+  const long q3 = g * M.fl[2].n + static_cast<long>(k) * M.fl[2].plane - M.fl[2].org;
   const double *w = ca.w + static_cast<long>(g) * NHYDRO * n + k * pc;
   const double *b = ca.bcc + static_cast<long>(g) * 3 * n + k * pc;
   MarchPlane P;
   P.w1 = ldb(ca.wx1 + q1, o1);
   P.e2x1 = ldb(ca.e2x1 + q1, o1);
   P.e3x1 = ldb(ca.e3x1 + q1, o1);
-  P.w2 = ldb(ca.wx2 + q2, oc);
-  P.e1x2 = ldb(ca.e1x2 + q2, oc);
-  P.e3x2 = ldb(ca.e3x2 + q2, oc);
-  P.w3 = ldb(ca.wx3 + q3, oc);
-  P.e1x3 = ldb(ca.e1x3 + q3, oc);
-  P.e2x3 = ldb(ca.e2x3 + q3, oc);
+  P.w2 = ldb(ca.wx2 + q2, o2);
+  P.e1x2 = ldb(ca.e1x2 + q2, o2);
+  P.e3x2 = ldb(ca.e3x2 + q2, o2);
+  P.w3 = ldb(ca.wx3 + q3, o2);
+  P.e1x3 = ldb(ca.e1x3 + q3, o2);
+  P.e2x3 = ldb(ca.e2x3 + q3, o2);
   P.vx = ldb(w + IVX * n, oc);
   P.vy = ldb(w + IVY * n, oc);
   P.vz = ldb(w + IVZ * n, oc);
@@ -1024,9 +1044,11 @@ __device__ __forceinline__ void corner_march(const MeshK &M, const CornerArgs &c
   const bool live = t < ncs && i <= iend && j <= jend;
   const bool act = live && ri > 0 && rj > 0;
   const unsigned oc = 8u * static_cast<unsigned>(j * M.nc1 + i);
-  const unsigned o1 = 8u * static_cast<unsigned>(j * (M.nc1 + 1) + i);
+  const unsigned o1 = 8u * static_cast<unsigned>(j * M.fl[0].row + i);
+  const unsigned o2 = 8u * static_cast<unsigned>(j * M.fl[1].row + i);
+  const unsigned oe = 8u * static_cast<unsigned>(j * (M.nc1 + 1) + i);
   MarchPlane C{}, N{};
-  if (live) C = march_load(M, ca, g, k0 - 1, oc, o1);
+  if (live) C = march_load(M, ca, g, k0 - 1, oc, o1, o2);
   // plane k-1: own face values, cell-centred E1 of this cell and one row down, E2 of this
   // cell and one column left
   double w1p = 0.0, w2p = 0.0, e12p = 0.0, e21p = 0.0, c0p = 0.0, c0jp = 0.0, c1p = 0.0;
@@ -1054,7 +1076,7 @@ __device__ __forceinline__ void corner_march(const MeshK &M, const CornerArgs &c
       S[7 * ncs + t] = cc0;
       S[8 * ncs + t] = cc1;
       S[9 * ncs + t] = cc2;
-      if (k + 1 < k1) N = march_load(M, ca, g, k + 1, oc, o1);
+      if (k + 1 < k1) N = march_load(M, ca, g, k + 1, oc, o1, o2);
     }
     __syncthreads();
     if (act) {
@@ -1083,7 +1105,7 @@ __device__ __forceinline__ void corner_march(const MeshK &M, const CornerArgs &c
           return sel(jj < j, sel(ii < i, cc2d, cc2j), sel(ii < i, cc2i, cc2));
         };
         auto out = [&](int comp, double v) {
-          unsigned c = oc, f = o1;
+          unsigned c = oc, f = oe;
           asm volatile("" : "+v"(c), "+v"(f));
           if (comp == 0)
             stb(ca.e1 + static_cast<long>(g) * M.ne1 + k * (static_cast<long>(M.nc2 + 1) * M.nc1),
@@ -1229,6 +1251,7 @@ __device__ __forceinline__ double emf1(const MeshK &M, const double *e, int g, i
 // copies are written afterwards by the exchange kernel (k_ghost).
 // first_stage: out = (0 + 1*base) - wght*div F   (u1 zeroed, delta = 1, then swapped)
 // otherwise:   out = base - wght*div F           (in place allowed: out == base)
+template <bool PACKED>
 __device__ __forceinline__ void update_cell_u(const MeshK &M, int g, int k, int j, int i,
                                               const double *base, double *out,
                                               const double *__restrict__ f1,
@@ -1242,16 +1265,19 @@ __device__ __forceinline__ void update_cell_u(const MeshK &M, int g, int k, int 
   const double vol = dx1[i] * dx2[j] * dx3[k];
   const long c = cidx(M, k, j, i);
   const long b0 = static_cast<long>(g) * NHYDRO * M.ncell;
-  const double *F1 = f1 + static_cast<long>(g) * NHYDRO * M.nf1;
-  const double *F2 = f2 + static_cast<long>(g) * NHYDRO * M.nf2;
-  const double *F3 = f3 + static_cast<long>(g) * NHYDRO * M.nf3;
-  const long x1 = f1idx(M, k, j, i), x2 = f2idx(M, k, j, i), x3 = f3idx(M, k, j, i);
-  const long sx2 = M.nc1, sx3 = static_cast<long>(M.nc2) * M.nc1;
+  const FaceLayout &L2 = M.fl[PACKED ? 0 : 1], &L3 = M.fl[PACKED ? 0 : 2];
+  const long n1 = M.fl[0].n, n2 = L2.n, n3 = L3.n;
+  const double *F1 = f1 + static_cast<long>(g) * NHYDRO * n1;
+  const double *F2 = f2 + static_cast<long>(g) * NHYDRO * n2;
+  const double *F3 = f3 + static_cast<long>(g) * NHYDRO * n3;
+  const long x1 = foidx<0>(M, k, j, i), x2 = foidx<PACKED ? 0 : 1>(M, k, j, i);
+  const long x3 = foidx<PACKED ? 0 : 2>(M, k, j, i);
+  const long sx2 = L2.row, sx3 = L3.plane;
 #pragma unroll
   for (int n = 0; n < NHYDRO; ++n) {
-    double dflx = (a1 * F1[n * M.nf1 + x1 + 1] - a1 * F1[n * M.nf1 + x1]);
-    dflx += (a2 * F2[n * M.nf2 + x2 + sx2] - a2 * F2[n * M.nf2 + x2]);
-    dflx += (a3 * F3[n * M.nf3 + x3 + sx3] - a3 * F3[n * M.nf3 + x3]);
+    double dflx = (a1 * F1[n * n1 + x1 + 1] - a1 * F1[n * n1 + x1]);
+    dflx += (a2 * F2[n * n2 + x2 + sx2] - a2 * F2[n * n2 + x2]);
+    dflx += (a3 * F3[n * n3 + x3 + sx3] - a3 * F3[n * n3 + x3]);
     double u0 = base[b0 + n * M.ncell + c];
     if (first_stage) u0 = 0.0 + 1.0 * u0;
     out[b0 + n * M.ncell + c] = u0 - wght * dflx / vol;
@@ -1321,7 +1347,7 @@ __device__ __forceinline__ void update_body(const MeshK &M, const UpdateArgs &a,
   const double wght = beta * dt;
   const bool ci = i <= M.ie, cj = j <= M.je, ck = k <= M.ke;
   if (do_u && ci && cj && ck)
-    update_cell_u(M, g, k, j, i, a.ubase, a.uout, a.f1, a.f2, a.f3, wght, first_stage);
+    update_cell_u<true>(M, g, k, j, i, a.ubase, a.uout, a.f1, a.f2, a.f3, wght, first_stage);
   if (cj && ck)
     update_face_b<0>(M, g, k, j, i, a.bin[0], a.bout[0], a.e1, a.e2, a.e3, wght, first_stage);
   if (ci && ck)
@@ -2094,7 +2120,7 @@ __global__ void __launch_bounds__(WG) k_blk_update(MeshK M, UpdateArgs a, double
   if (!map_kind(M, KK_UPDATE, blockIdx.x, gridDim.x, TileK{0, 0, 0}, g, i, j, k)) return;
   const bool ci = i <= M.ie, cj = j <= M.je, ck = k <= M.ke;
   if ((what & 1) && ci && cj && ck)
-    update_cell_u(M, g, k, j, i, a.uout, a.uout, a.f1, a.f2, a.f3, wght, 0);
+    update_cell_u<false>(M, g, k, j, i, a.uout, a.uout, a.f1, a.f2, a.f3, wght, 0);
   if (what & 2) {
     if (cj && ck)
       update_face_b<0>(M, g, k, j, i, a.bout[0], a.bout[0], a.e1, a.e2, a.e3, wght, 0);
@@ -2253,6 +2279,12 @@ __device__ __forceinline__ refops::View face_view(const MeshK &M, double *p, int
   const long nf = (c == 0) ? M.nf1 : ((c == 1) ? M.nf2 : M.nf3);
   return refops::View{p + static_cast<long>(g) * nf, M.nc2 + (c == 1), M.nc1 + (c == 0)};
 }
+__device__ __forceinline__ refops::View flux_view(const MeshK &M, double *p, int g, int n,
+                                                  int c) {
+  const FaceLayout L = (c == 0) ? M.fl[0] : ((c == 1) ? M.fl[1] : M.fl[2]);
+  return refops::View{p + (static_cast<long>(g) * NHYDRO + n) * L.n - L.org, L.plane / L.row,
+                      L.row};
+}
 __device__ __forceinline__ refops::View edge_view(const MeshK &M, const double *p, int g,
                                                   int c) {
   const long ne = (c == 0) ? M.ne1 : ((c == 1) ? M.ne2 : M.ne3);
@@ -2328,9 +2360,7 @@ __device__ __forceinline__ void smr_bcc_p2c(const MeshK &M, const SmrArgs &a, in
 // (k, j, i) (LoadFluxBoundaryBufferToCoarser, flux_correction_cc.cpp:77-166).
 __device__ __forceinline__ double smr_flux_restrict(const MeshK &M, const SmrArgs &a, int dir,
                                                     int src, int n, int k, int j, int i) {
-  const long nf = (dir == 0) ? M.nf1 : ((dir == 1) ? M.nf2 : M.nf3);
-  const refops::View f{a.flux[dir] + (static_cast<long>(src) * NHYDRO + n) * nf,
-                       M.nc2 + (dir == 1), M.nc1 + (dir == 0)};
+  const refops::View f = flux_view(M, a.flux[dir], src, n, dir);
   const double *d1 = ctab(M, src, 0), *d2 = ctab(M, src, 1), *d3 = ctab(M, src, 2);
   if (dir == 0) {
     const double amm = d2[j] * d3[k], amp = d2[j + 1] * d3[k];
@@ -2433,9 +2463,7 @@ __global__ void __launch_bounds__(smrplan::CHUNK_THREADS) k_smr(MeshK M, SmrArgs
           smr_bcc_p2c(M, a, g, k, j, i);
           break;
         case smrplan::FLUX_RESTRICT: {
-          const long nf = (c == 0) ? M.nf1 : ((c == 1) ? M.nf2 : M.nf3);
-          const refops::View f{a.flux[c] + (static_cast<long>(g) * NHYDRO + n) * nf,
-                               M.nc2 + (c == 1), M.nc1 + (c == 0)};
+          const refops::View f = flux_view(M, a.flux[c], g, n, c);
           f(k, j, i) = smr_flux_restrict(M, a, c, st.src, n, sk, sj, si);
           break;
         }
@@ -2528,6 +2556,10 @@ struct ath_mesh {
   std::vector<Rec> prof_rec;
   double prof_ms[64] = {0};
   long prof_cnt[64] = {0};
+
+  // entries of per-face registers outside the packed arrays, as the caller last set them
+  std::map<std::pair<int, int>, std::vector<double>> unpacked;
+  std::mutex unpacked_mutex;
 
   int alloc(double **p, long n) {
     HIPCHK(hipMalloc(reinterpret_cast<void **>(p), sizeof(double) * n));
@@ -2635,6 +2667,63 @@ constexpr TileK TILES[NTILES] = {{0, 0, 0}, {64, 4, 1}, {32, 8, 1}, {16, 16, 1},
 bool tile_ok(int kind, int t) { return TILES[t].tx >= 0 || kind == KK_CORNER; }
 // A single mesh also runs the flux kernel's z-march (k_flux_zm); ensembles do not.
 bool mesh_tile_ok(int kind, int t) { return tile_ok(kind, t) || kind == KK_FLUX; }
+
+// Layouts of the per-face outputs.  public: the extents of the face fields, as a MeshBlock
+// holds them (the per-block entries).  packed: all three directions over the flux kernel's
+// box [is-1,ie+1] x [js-1,je+1] x [ks-1,ke+1] and nothing else, each component padded to
+// whole cache lines, so that a work-group's 256 consecutive cells write whole lines.  With
+// the unused ends of each row in between, nearly every second line is written in part, and
+// such lines take HBM 1.5 to 1.8 times as long: the 24 arrays alone of 64 blocks of 32^3
+// cells 265 against 153 us (a kernel that only copies).  DC fluxes over 64 blocks of 64^3
+// cells 1.99 -> 1.76 ms, corner EMFs 0.70 -> 0.66 (64 of 32^3: 120 -> 106 us; a refined mesh
+// of 16^3 blocks: 91 -> 69); the update 1.20 -> 1.23 ms.
+void public_faces(MeshK &M) {
+  const long nf[3] = {M.nf1, M.nf2, M.nf3};
+  for (int d = 0; d < 3; ++d) {
+    M.fl[d].row = M.nc1 + (d == 0);
+    M.fl[d].plane = M.fl[d].row * (M.nc2 + (d == 1));
+    M.fl[d].org = 0;
+    M.fl[d].n = nf[d];
+  }
+  M.packed = 0;
+}
+
+void pack_faces(MeshK &M) {
+  for (int d = 0; d < 3; ++d) {
+    M.fl[d].row = M.nx1 + 2;
+    M.fl[d].plane = (M.nx1 + 2) * (M.nx2 + 2);
+    M.fl[d].org = static_cast<long>(M.ks - 1) * M.fl[d].plane +
+                  static_cast<long>(M.js - 1) * M.fl[d].row + (M.is - 1);
+    M.fl[d].n = (static_cast<long>(M.fl[d].plane) * (M.nx3 + 2) + 15) / 16 * 16;
+  }
+  M.packed = 1;
+}
+
+// The per-face output register `what` as (direction, components), or direction -1.
+int face_register(int what, int *ncomp) {
+  *ncomp = (what >= ATH_FLUX1 && what <= ATH_FLUX3) ? NHYDRO : 1;
+  if (what >= ATH_FLUX1 && what <= ATH_FLUX3) return what - ATH_FLUX1;
+  if (what >= ATH_WGHT1 && what <= ATH_WGHT3) return what - ATH_WGHT1;
+  return -1;
+}
+
+// Moves the faces that the flux kernel computes along d between one block's public array
+// and its packed one.
+void copy_faces(const MeshK &M, int d, int ncomp, double *pub, double *packed, bool pack) {
+  MeshK P = M;
+  public_faces(P);
+  const FaceLayout &A = P.fl[d], &B = M.fl[d];
+  for (int n = 0; n < ncomp; ++n)
+    for (int k = M.ks - (d != 2); k <= M.ke + 1; ++k)
+      for (int j = M.js - (d != 1); j <= M.je + 1; ++j) {
+        const int i0 = M.is - (d != 0);
+        double *a = pub + n * A.n + static_cast<long>(k) * A.plane + j * A.row + i0;
+        double *b = packed + n * B.n + static_cast<long>(k) * B.plane + j * B.row + i0 - B.org;
+        const size_t bytes = sizeof(double) * (M.ie + 2 - i0);
+        if (pack) std::memcpy(b, a, bytes);
+        else std::memcpy(a, b, bytes);
+      }
+}
 
 // The z-march tile of a corner launch: segments of 2 planes (tile option 6) or 4 (7), one
 // where that would leave the GPU's 256 CUs short of three work-groups each.  Low segments
@@ -3589,6 +3678,7 @@ int mesh_build(const ath_mesh_desc *desc, const std::vector<smrplan::BlockInfo> 
   M.ne1 = static_cast<long>(M.nc3 + 1) * (M.nc2 + 1) * M.nc1;
   M.ne2 = static_cast<long>(M.nc3 + 1) * M.nc2 * (M.nc1 + 1);
   M.ne3 = static_cast<long>(M.nc3) * (M.nc2 + 1) * (M.nc1 + 1);
+  pack_faces(M);
   M.coff[0] = 0;
   M.coff[1] = 3 * M.nc1;
   M.coff[2] = 3 * (M.nc1 + M.nc2);
@@ -3688,16 +3778,16 @@ int mesh_build(const ath_mesh_desc *desc, const std::vector<smrplan::BlockInfo> 
   for (int q = 0; q < 3 && !rc; ++q) {
     rc |= m->alloc(&m->b[q], nf[q] * nb);
     rc |= m->alloc(&m->bb[q], nf[q] * nb);
-    rc |= m->alloc(&m->flux[q], NHYDRO * nf[q] * nb);
-    rc |= m->alloc(&m->wx[q], nf[q] * nb);
+    rc |= m->alloc(&m->flux[q], NHYDRO * M.fl[q].n * nb);
+    rc |= m->alloc(&m->wx[q], M.fl[q].n * nb);
   }
   if (!rc) {
-    rc |= m->alloc(&m->e2x1, nf[0] * nb);
-    rc |= m->alloc(&m->e3x1, nf[0] * nb);
-    rc |= m->alloc(&m->e1x2, nf[1] * nb);
-    rc |= m->alloc(&m->e3x2, nf[1] * nb);
-    rc |= m->alloc(&m->e1x3, nf[2] * nb);
-    rc |= m->alloc(&m->e2x3, nf[2] * nb);
+    rc |= m->alloc(&m->e2x1, M.fl[0].n * nb);
+    rc |= m->alloc(&m->e3x1, M.fl[0].n * nb);
+    rc |= m->alloc(&m->e1x2, M.fl[1].n * nb);
+    rc |= m->alloc(&m->e3x2, M.fl[1].n * nb);
+    rc |= m->alloc(&m->e1x3, M.fl[2].n * nb);
+    rc |= m->alloc(&m->e2x3, M.fl[2].n * nb);
     rc |= m->alloc(&m->e[0], M.ne1 * nb);
     rc |= m->alloc(&m->e[1], M.ne2 * nb);
     rc |= m->alloc(&m->e[2], M.ne3 * nb);
@@ -3853,6 +3943,24 @@ int ath_gpu_set_block(ath_mesh_t m, int gid, int what, const double *host) {
   long n;
   double **pool;
   if (block_count(m, what, &n, &pool)) return 1;
+  int nc;
+  const int d = face_register(what, &nc);
+  if (d >= 0) try {
+    // the computed faces to the packed array; the others are kept for ath_gpu_get_block
+    const long np = nc * m->M.fl[d].n;
+    std::vector<double> packed(np, 0.0), rest(host, host + n);
+    copy_faces(m->M, d, nc, rest.data(), packed.data(), true);
+    {
+      const std::lock_guard<std::mutex> lock(m->unpacked_mutex);
+      m->unpacked[{what, gid}] = std::move(rest);
+    }
+    HIPCHK(hipMemcpyAsync(*pool + gid * np, packed.data(), sizeof(double) * np,
+                          hipMemcpyHostToDevice, m->stream));
+    HIPCHK(hipStreamSynchronize(m->stream));
+    return 0;
+  } catch (const std::exception &e) {
+    return fail(e.what());
+  }
   HIPCHK(hipMemcpyAsync(*pool + static_cast<long>(gid) * n, host, sizeof(double) * n,
                         hipMemcpyHostToDevice, m->stream));
   HIPCHK(hipStreamSynchronize(m->stream));
@@ -3865,6 +3973,25 @@ int ath_gpu_get_block(ath_mesh_t m, int gid, int what, double *host) {
   long n;
   double **pool;
   if (block_count(m, what, &n, &pool)) return 1;
+  int nc;
+  const int d = face_register(what, &nc);
+  if (d >= 0) try {
+    const long np = nc * m->M.fl[d].n;
+    std::vector<double> packed(np);
+    HIPCHK(hipMemcpyAsync(packed.data(), *pool + gid * np, sizeof(double) * np,
+                          hipMemcpyDeviceToHost, m->stream));
+    HIPCHK(hipStreamSynchronize(m->stream));
+    {
+      const std::lock_guard<std::mutex> lock(m->unpacked_mutex);
+      const auto rest = m->unpacked.find({what, gid});
+      if (rest != m->unpacked.end()) std::copy(rest->second.begin(), rest->second.end(), host);
+      else std::fill(host, host + n, 0.0);
+    }
+    copy_faces(m->M, d, nc, host, packed.data(), false);
+    return 0;
+  } catch (const std::exception &e) {
+    return fail(e.what());
+  }
   HIPCHK(hipMemcpyAsync(host, *pool + static_cast<long>(gid) * n, sizeof(double) * n,
                         hipMemcpyDeviceToHost, m->stream));
   HIPCHK(hipStreamSynchronize(m->stream));
@@ -4592,6 +4719,7 @@ int ath_gpu_block_create(const ath_block_desc *d, ath_block_t *out) {
   M.ne1 = static_cast<long>(M.nc3 + 1) * (M.nc2 + 1) * M.nc1;
   M.ne2 = static_cast<long>(M.nc3 + 1) * M.nc2 * (M.nc1 + 1);
   M.ne3 = static_cast<long>(M.nc3) * (M.nc2 + 1) * (M.nc1 + 1);
+  public_faces(M);
   M.coff[0] = 0;
   M.coff[1] = 3 * M.nc1;
   M.coff[2] = 3 * (M.nc1 + M.nc2);

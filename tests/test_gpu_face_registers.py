@@ -1,0 +1,62 @@
+"""GPU checks of the per-face registers (fluxes and CT weights), which a mesh keeps packed
+over the computed faces only: what a caller sets comes back whole, the computed faces hold
+the oracle's values in the array extents the caller sees, and the rest stays as set."""
+import numpy as np
+import pytest
+
+from athena_amd.gpu import GpuMesh
+from athena_amd.mesh import MeshDesc
+from athena_amd.pgen.blast import Blast
+from oracle_bind import OracleMesh
+
+pytestmark = pytest.mark.gpu
+REGS = ("flux1", "flux2", "flux3", "wght1", "wght2", "wght3")
+
+
+def _mesh(nx, bnx, ng):
+    m = MeshDesc(nx=nx, bnx=bnx, xmin=(-0.5,) * 3, xmax=(0.5,) * 3, gamma=5.0 / 3.0, cfl=0.3,
+                 xorder=3 if ng > 2 else 2, ng=ng, rsolver="hlld")
+    return m, Blast(m)
+
+
+def _shape(m, reg):
+    d = int(reg[-1]) - 1
+    ext = [m.bnx[q] + 2 * m.ng + (q == d) for q in (2, 1, 0)]
+    return ([5] if reg.startswith("flux") else []) + ext
+
+
+@pytest.mark.parametrize("nx,bnx,ng", [((4, 4, 4), (2, 2, 2), 2), ((10, 6, 7), (5, 3, 7), 2),
+                                       ((17, 16, 5), (17, 8, 5), 3), ((15, 8, 5), (15, 4, 5), 4)])
+def test_face_registers(nx, bnx, ng):
+    m, ic = _mesh(nx, bnx, ng)
+    print("case face registers", nx, bnx, ng, flush=True)
+    d = GpuMesh(m)
+    rng = np.random.default_rng(7)
+    put = {}
+    for reg in REGS:
+        for g in (0, m.nblocks - 1):
+            put[g, reg] = rng.standard_normal(_shape(m, reg))
+            d.set(g, reg, put[g, reg])
+    for (g, reg), a in put.items():
+        assert np.array_equal(d.get(g, reg).reshape(a.shape), a), (g, reg)
+
+    blocks = [ic.block(g) for g in range(m.nblocks)]
+    o = OracleMesh(m)
+    o.load(blocks)
+    o.initialize(1e300)
+    o.run(2, 1e300)
+    d.load(blocks)
+    d.initialize(1e300)
+    d.run(2)
+    lo, n = ng, m.bnx
+    for (g, reg), a in put.items():
+        x = int(reg[-1]) - 1
+        got = d.get(g, reg).reshape(a.shape)
+        want = o.get(g, reg).reshape(a.shape)
+        # the faces of active cells; then everything the flux kernel does not compute
+        act = tuple(slice(lo, lo + n[q] + (q == x)) for q in (2, 1, 0))
+        assert np.array_equal(got[(...,) + act], want[(...,) + act]), (g, reg)
+        comp = tuple(slice(lo - (q != x), lo + n[q] + 1) for q in (2, 1, 0))
+        rest = np.ones(a.shape, bool)
+        rest[(...,) + comp] = False
+        assert np.array_equal(got[rest], a[rest]), (g, reg)
