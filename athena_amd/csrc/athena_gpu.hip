@@ -22,6 +22,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -310,18 +311,35 @@ struct FaceOut {
   double *flx, *ey, *ez, *wct;
 };
 
-template <int DIR, int ORDER, int RS>
+// The same registers stored streaming, past the L2 caches: for sets of outputs larger than
+// those, which the next kernels read from memory either way, so that the rows a launch's
+// stencils share stay cached.  At 256^3 (64 blocks of 64^3 cells) PLM fluxes 2.36 -> 2.27 ms,
+// DC 1.76 -> 1.63, corner EMFs 0.66 -> 0.64; 128^3 (32^3) corner EMFs 106 -> 90 us; a mesh
+// of 32^3 cells (9 MB of outputs), streamed: update 15.2 -> 16.9 us.  The kind of store is
+// the launch's, not chosen per store: a branch around each took PPM fluxes 659 -> 693 us.
+struct FaceOutStream : FaceOut {
+  __device__ explicit FaceOutStream(const FaceOut &o) : FaceOut(o) {}
+};
+template <bool STREAM>
+using FaceOutOf = std::conditional_t<STREAM, FaceOutStream, FaceOut>;
+
+__device__ __forceinline__ void face_put(const FaceOut &, double *p, double v) { *p = v; }
+__device__ __forceinline__ void face_put(const FaceOutStream &, double *p, double v) {
+  __builtin_nontemporal_store(v, p);
+}
+
+template <int DIR, int ORDER, int RS, class FO>
 __device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, int i,
-                                           double *wl, double *wr, const FaceOut &o,
+                                           double *wl, double *wr, const FO &o,
                                            double dt, bool emit, double *fx);
 
 // One interface along DIR at face (k, j, i) of block g: reconstruction, the Riemann
 // solver, and the face EMFs and CT weight of that face written to o (when emit); the five
 // fluxes are returned in fx[] in conserved order (IDN, IM1, IM2, IM3, IEN).
-template <int DIR, int ORDER, int RS>
+template <int DIR, int ORDER, int RS, class FO>
 __device__ __forceinline__ void face_flux(const MeshK &M, int g, int k, int j, int i,
                                           const double *__restrict__ wb,
-                                          const double *__restrict__ bb, const FaceOut &o,
+                                          const double *__restrict__ bb, const FO &o,
                                           double dt, bool emit, double *fx) {
   const long s = (DIR == 0) ? 1 : ((DIR == 1) ? M.nc1 : static_cast<long>(M.nc1) * M.nc2);
   const long c = cidx(M, k, j, i);
@@ -382,9 +400,9 @@ __device__ __forceinline__ void face_flux(const MeshK &M, int g, int k, int j, i
 // The rest of one interface once its states are reconstructed: the primitive floors
 // (PPM), the Riemann solver, the fluxes returned in fx[] in conserved order, and the face
 // EMFs and CT weight written to o (when emit).  wl and wr are in the rotated order of DIR.
-template <int DIR, int ORDER, int RS>
+template <int DIR, int ORDER, int RS, class FO>
 __device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, int i,
-                                           double *wl, double *wr, const FaceOut &o,
+                                           double *wl, double *wr, const FO &o,
                                            double dt, bool emit, double *fx) {
   constexpr int ivx = IVX + DIR;
   constexpr int ivy = IVX + ((ivx - IVX) + 1) % 3;
@@ -418,27 +436,27 @@ __device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, 
   fx[IEN] = f[IEN];
   if (emit) {
     const long q = static_cast<long>(g) * M.fl[DIR].n + foidx<DIR>(M, k, j, i);
-    o.ey[q] = -f[IBY];
-    o.ez[q] = f[IBZ];
+    face_put(o, &o.ey[q], -f[IBY]);
+    face_put(o, &o.ez[q], f[IBZ]);
     const double dxw = ct[fc];
-    o.wct[q] = ct_weight(f[IDN], wl[IDN], wr[IDN], dxw, dt);
+    face_put(o, &o.wct[q], ct_weight(f[IDN], wl[IDN], wr[IDN], dxw, dt));
   }
 }
 
-template <int DIR>
+template <int DIR, class FO>
 __device__ __forceinline__ void store_flux(const MeshK &M, int g, int k, int j, int i,
-                                           const FaceOut &o, const double *fx) {
+                                           const FO &o, const double *fx) {
   const long nf = M.fl[DIR].n;
   double *fb = o.flx + static_cast<long>(g) * NHYDRO * nf + foidx<DIR>(M, k, j, i);
 #pragma unroll
-  for (int n = 0; n < NHYDRO; ++n) fb[n * nf] = fx[n];
+  for (int n = 0; n < NHYDRO; ++n) face_put(o, &fb[n * nf], fx[n]);
 }
 
 // face_flux with the fluxes written to Hydro::flux[DIR] (o.flx) as well.
-template <int DIR, int ORDER, int RS>
+template <int DIR, int ORDER, int RS, class FO>
 __device__ __forceinline__ void flux_face(const MeshK &M, int g, int k, int j, int i,
                                           const double *__restrict__ wb,
-                                          const double *__restrict__ bb, const FaceOut &o,
+                                          const double *__restrict__ bb, const FO &o,
                                           double dt) {
   double fx[NHYDRO];
   face_flux<DIR, ORDER, RS>(M, g, k, j, i, wb, bb, o, dt, true, fx);
@@ -469,10 +487,10 @@ __global__ void __launch_bounds__(WG) k_flux(MeshK M, const double *__restrict__
 // One thread per cell of [is-1,ie+1]x[js-1,je+1]x[ks-1,ke+1]; each computes the faces on
 // its low sides that lie in the reference's loop ranges (calculate_fluxes.cpp:68-76,
 // 176-182, 299-302).
-template <int ORDER, int RS>
+template <int ORDER, int RS, class FO>
 __device__ __forceinline__ void flux3_body(const MeshK &M, const double *__restrict__ w,
-                                           const double *__restrict__ bcc, const FaceOut &o1,
-                                           const FaceOut &o2, const FaceOut &o3, double dt,
+                                           const double *__restrict__ bcc, const FO &o1,
+                                           const FO &o2, const FO &o3, double dt,
                                            int lw, int nwg, TileK T) {
   int g, i, j, k;
   if (!map_kind(M, KK_FLUX, lw, nwg, T, g, i, j, k)) return;
@@ -483,22 +501,23 @@ __device__ __forceinline__ void flux3_body(const MeshK &M, const double *__restr
   } else if (M.packed) {   // the row's unused first entry: complete its cache line
     const long q = static_cast<long>(g) * M.fl[0].n + foidx<0>(M, k, j, i);
     const double zero[NHYDRO] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    o1.ey[q] = 0.0;
-    o1.ez[q] = 0.0;
-    o1.wct[q] = 0.0;
+    face_put(o1, &o1.ey[q], 0.0);
+    face_put(o1, &o1.ez[q], 0.0);
+    face_put(o1, &o1.wct[q], 0.0);
     store_flux<0>(M, g, k, j, i, o1, zero);
   }
   if (j >= M.js) flux_face<1, ORDER, RS>(M, g, k, j, i, wb, bb, o2, dt);
   if (k >= M.ks) flux_face<2, ORDER, RS>(M, g, k, j, i, wb, bb, o3, dt);
 }
 
-template <int ORDER, int RS>
+template <int ORDER, int RS, bool STREAM>
 __global__ void __launch_bounds__(WG) k_flux3(MeshK M, const double *__restrict__ w,
                                                const double *__restrict__ bcc, FaceOut o1,
                                                FaceOut o2, FaceOut o3,
                                                const Clock *__restrict__ clk, TileK T) {
-  flux3_body<ORDER, RS>(M, w, bcc, o1, o2, o3, clk->dt, xcd_logical_wg(M.xcd_remap & XCD_FLUX),
-                        gridDim.x, T);
+  using FO = FaceOutOf<STREAM>;
+  flux3_body<ORDER, RS>(M, w, bcc, FO(o1), FO(o2), FO(o3), clk->dt,
+                        xcd_logical_wg(M.xcd_remap & XCD_FLUX), gridDim.x, T);
 }
 
 // Reconstruction of cell (k, j, i) along DIR: its low-face value qm[v] and high-face value
@@ -1916,14 +1935,15 @@ __device__ __forceinline__ int2 ens_item(const int2 *__restrict__ map, int v) {
   return make_int2(__builtin_amdgcn_readfirstlane(mw.x), __builtin_amdgcn_readfirstlane(mw.y));
 }
 
-template <int ORDER, int RS>
+template <int ORDER, int RS, bool STREAM>
 __global__ void __launch_bounds__(WG) k_flux3_ens(const EnsMember *__restrict__ E,
                                                    const int2 *__restrict__ map, int nwork) {
   for (int v = blockIdx.x; v < nwork; v += gridDim.x) {
     const int2 mw = ens_item(map, v);
     const EnsMember &e = E[mw.x];
-    flux3_body<ORDER, RS>(e.M, e.w, e.bcc, e.fo[0], e.fo[1], e.fo[2], e.clk->dt, mw.y,
-                          e.nwg[0], e.tile[0]);
+    using FO = FaceOutOf<STREAM>;
+    flux3_body<ORDER, RS>(e.M, e.w, e.bcc, FO(e.fo[0]), FO(e.fo[1]), FO(e.fo[2]), e.clk->dt,
+                          mw.y, e.nwg[0], e.tile[0]);
   }
 }
 
@@ -2699,6 +2719,13 @@ void pack_faces(MeshK &M) {
   M.packed = 1;
 }
 
+// Bytes of a mesh's packed per-face outputs: eight for each of the three faces of a cell.
+double face_bytes(const MeshK &M) { return 24.0 * sizeof(double) * M.fl[0].n * M.nblocks; }
+
+// Whether a flux launch that writes this much streams it: more than the 4 MB of L2 in each
+// of the 8 XCDs.
+bool stream_faces(double bytes) { return bytes > 32.0 * (1 << 20); }
+
 // The per-face output register `what` as (direction, components), or direction -1.
 int face_register(int what, int *ncomp) {
   *ncomp = (what >= ATH_FLUX1 && what <= ATH_FLUX3) ? NHYDRO : 1;
@@ -2822,9 +2849,16 @@ int launch_flux_args(ath_mesh *m, int order, const double *w, const double *bcc,
                                                     (WG / 64)))
                        : kind_grid(m, KK_FLUX);
   ProfScope ps(m, KID_FLUX3 + (order - 1));
+  const bool stream = stream_faces(face_bytes(M));
 #define LF(O, R)                                                                          \
-  hipLaunchKernelGGL((k_flux3<O, R>), grid, dim3(WG), 0, m->stream, M, w, bcc, fo[0], fo[1], \
-                     fo[2], m->clk, T)
+  do {                                                                                    \
+    if (stream)                                                                           \
+      hipLaunchKernelGGL((k_flux3<O, R, true>), grid, dim3(WG), 0, m->stream, M, w, bcc,  \
+                         fo[0], fo[1], fo[2], m->clk, T);                                 \
+    else                                                                                  \
+      hipLaunchKernelGGL((k_flux3<O, R, false>), grid, dim3(WG), 0, m->stream, M, w, bcc, \
+                         fo[0], fo[1], fo[2], m->clk, T);                                 \
+  } while (0)
 #define LZ(O, R)                                                                          \
   hipLaunchKernelGGL((k_flux_zm<O, R>), grid, dim3(WG), 0, m->stream, M, w, bcc, fo[0],   \
                      fo[1], fo[2], m->clk, T.tz)
@@ -3340,7 +3374,16 @@ int ens_launch_kind(ath_ensemble *e, int kind, int stg) {
   const int nw = e->nwork[kind];
   if (kind == KK_FLUX) {
     const int order = (stg == 1) ? 1 : e->xorder;
-#define LE(O, R) hipLaunchKernelGGL((k_flux3_ens<O, R>), g, dim3(WG), 0, e->stream, T, mp, nw)
+    double bytes = 0.0;
+    for (const auto *m : e->mem) bytes += face_bytes(m->M);
+    const bool stream = stream_faces(bytes);
+#define LE(O, R)                                                                             \
+  do {                                                                                       \
+    if (stream)                                                                              \
+      hipLaunchKernelGGL((k_flux3_ens<O, R, true>), g, dim3(WG), 0, e->stream, T, mp, nw);   \
+    else                                                                                     \
+      hipLaunchKernelGGL((k_flux3_ens<O, R, false>), g, dim3(WG), 0, e->stream, T, mp, nw);  \
+  } while (0)
 #define LE_O(R)                         \
   do {                                  \
     if (order == 1) LE(1, R);           \

@@ -4,7 +4,7 @@ the oracle's values in the array extents the caller sees, and the rest stays as 
 import numpy as np
 import pytest
 
-from athena_amd.gpu import GpuMesh
+from athena_amd.gpu import Ensemble, GpuMesh
 from athena_amd.mesh import MeshDesc
 from athena_amd.pgen.blast import Blast
 from oracle_bind import OracleMesh
@@ -60,3 +60,35 @@ def test_face_registers(nx, bnx, ng):
         rest = np.ones(a.shape, bool)
         rest[(...,) + comp] = False
         assert np.array_equal(got[rest], a[rest]), (g, reg)
+
+
+@pytest.mark.parametrize("bnx,nx,rsolver,xorder", [((16, 16, 16), (48, 48, 64), "hlld", 2),
+                                                   ((27, 16, 29), (54, 64, 58), "hlle", 3)])
+def test_streamed_faces(bnx, nx, rsolver, xorder):
+    """More than 32 MB of per-face outputs: the flux launches store them past the L2 caches.
+    A mesh by itself and, with a smaller one, in an ensemble."""
+    m = MeshDesc(nx=nx, bnx=bnx, xmin=(-0.5,) * 3, xmax=(0.5,) * 3, gamma=5.0 / 3.0, cfl=0.3,
+                 xorder=xorder, ng=xorder if xorder == 2 else 4, rsolver=rsolver)
+    print("case streamed faces", nx, bnx, rsolver, flush=True)
+    assert 24 * 8 * m.nblocks * np.prod([n + 2 for n in bnx]) > 32 * 2**20
+    blocks = [Blast(m).block(g) for g in range(m.nblocks)]
+    o = OracleMesh(m)
+    o.load(blocks)
+    o.initialize(1e300)
+    o.run(2, 1e300)
+    dev = [GpuMesh(m), GpuMesh(m)]
+    for d in dev:
+        d.load(blocks)
+        d.initialize(1e300)
+    dev[0].run(2)
+    small = MeshDesc(nx=bnx, bnx=bnx, xmin=(-0.5,) * 3, xmax=(0.5,) * 3, gamma=5.0 / 3.0,
+                     cfl=0.3, xorder=xorder, ng=m.ng, rsolver=rsolver)
+    s = GpuMesh(small)
+    s.load([Blast(small).block(0)])
+    s.initialize(1e300)
+    e = Ensemble([dev[1], s])
+    e.run(2)
+    for d in dev:
+        for g in range(m.nblocks):
+            for key in ("u", "b1", "b2", "b3"):
+                assert np.array_equal(d.get(g, key).ravel(), o.get(g, key).ravel()), (g, key)
