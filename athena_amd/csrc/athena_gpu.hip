@@ -333,6 +333,13 @@ __device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, 
                                            double *wl, double *wr, const FO &o,
                                            double dt, bool emit, double *fx);
 
+template <int DIR>
+__device__ __forceinline__ long bidx(const MeshK &M, int g, int k, int j, int i) {
+  if (DIR == 0) return static_cast<long>(g) * M.nf1 + f1idx(M, k, j, i);
+  if (DIR == 1) return static_cast<long>(g) * M.nf2 + f2idx(M, k, j, i);
+  return static_cast<long>(g) * M.nf3 + f3idx(M, k, j, i);
+}
+
 // One interface along DIR at face (k, j, i) of block g: reconstruction, the Riemann
 // solver, and the face EMFs and CT weight of that face written to o (when emit); the five
 // fluxes are returned in fx[] in conserved order (IDN, IM1, IM2, IM3, IEN).
@@ -397,32 +404,15 @@ __device__ __forceinline__ void face_flux(const MeshK &M, int g, int k, int j, i
   face_solve<DIR, ORDER, RS>(M, g, k, j, i, wl, wr, o, dt, emit, fx);
 }
 
-// The rest of one interface once its states are reconstructed: the primitive floors
-// (PPM), the Riemann solver, the fluxes returned in fx[] in conserved order, and the face
-// EMFs and CT weight written to o (when emit).  wl and wr are in the rotated order of DIR.
-template <int DIR, int ORDER, int RS, class FO>
-__device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, int i,
-                                           double *wl, double *wr, const FO &o,
-                                           double dt, bool emit, double *fx) {
+// The Riemann solver at one interface with normal field bx and cell width *dxw; see face_solve.
+template <int DIR, int RS, class FO>
+__device__ __forceinline__ void face_emit(const MeshK &M, int g, int k, int j, int i,
+                                          double *wl, double *wr, double bx,
+                                          const double *dxw, const FO &o, double dt,
+                                          bool emit, double *fx) {
   constexpr int ivx = IVX + DIR;
   constexpr int ivy = IVX + ((ivx - IVX) + 1) % 3;
   constexpr int ivz = IVX + ((ivx - IVX) + 2) % 3;
-  const int fc = (DIR == 0) ? i : ((DIR == 1) ? j : k);
-  const double *ct = ctab(M, g, DIR);
-  if (ORDER == 3) {   // ApplyPrimitiveFloors on both reconstructed states
-    wl[IDN] = (wl[IDN] > M.eos.dfloor) ? wl[IDN] : M.eos.dfloor;
-    wl[IPR] = (wl[IPR] > M.eos.pfloor) ? wl[IPR] : M.eos.pfloor;
-    wr[IDN] = (wr[IDN] > M.eos.dfloor) ? wr[IDN] : M.eos.dfloor;
-    wr[IPR] = (wr[IPR] > M.eos.pfloor) ? wr[IPR] : M.eos.pfloor;
-  }
-
-  long fi;
-  if (DIR == 0) fi = f1idx(M, k, j, i);
-  else if (DIR == 1) fi = f2idx(M, k, j, i);
-  else fi = f3idx(M, k, j, i);
-  const long nf = (DIR == 0) ? M.nf1 : ((DIR == 1) ? M.nf2 : M.nf3);
-  const double bx = o.bn[static_cast<long>(g) * nf + fi];
-
   double f[NWAVE];
   if (RS == 0) hlld(wl, wr, bx, M.eos, f);
   else if (RS == 1) hlle(wl, wr, bx, M.eos, f);
@@ -438,9 +428,27 @@ __device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, 
     const long q = static_cast<long>(g) * M.fl[DIR].n + foidx<DIR>(M, k, j, i);
     face_put(o, &o.ey[q], -f[IBY]);
     face_put(o, &o.ez[q], f[IBZ]);
-    const double dxw = ct[fc];
-    face_put(o, &o.wct[q], ct_weight(f[IDN], wl[IDN], wr[IDN], dxw, dt));
+    face_put(o, &o.wct[q], ct_weight(f[IDN], wl[IDN], wr[IDN], *dxw, dt));
   }
+}
+
+// The rest of one interface once its states are reconstructed: the primitive floors
+// (PPM), the Riemann solver, the fluxes returned in fx[] in conserved order, and the face
+// EMFs and CT weight written to o (when emit).  wl and wr are in the rotated order of DIR.
+template <int DIR, int ORDER, int RS, class FO>
+__device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, int i,
+                                           double *wl, double *wr, const FO &o,
+                                           double dt, bool emit, double *fx) {
+  const int fc = (DIR == 0) ? i : ((DIR == 1) ? j : k);
+  if (ORDER == 3) {   // ApplyPrimitiveFloors on both reconstructed states
+    wl[IDN] = (wl[IDN] > M.eos.dfloor) ? wl[IDN] : M.eos.dfloor;
+    wl[IPR] = (wl[IPR] > M.eos.pfloor) ? wl[IPR] : M.eos.pfloor;
+    wr[IDN] = (wr[IDN] > M.eos.dfloor) ? wr[IDN] : M.eos.dfloor;
+    wr[IPR] = (wr[IPR] > M.eos.pfloor) ? wr[IPR] : M.eos.pfloor;
+  }
+
+  const double bx = o.bn[bidx<DIR>(M, g, k, j, i)];
+  face_emit<DIR, RS>(M, g, k, j, i, wl, wr, bx, ctab(M, g, DIR) + fc, o, dt, emit, fx);
 }
 
 template <int DIR, class FO>
@@ -484,6 +492,67 @@ __global__ void __launch_bounds__(WG) k_flux(MeshK M, const double *__restrict__
                             bcc + static_cast<long>(g) * 3 * M.ncell, o, clk->dt);
 }
 
+// Donor-cell faces: the inputs of the low face of a cell along one direction, other than
+// the cell's own values (w, bcc): the values of the cell below, the normal field and the
+// cell width.  In bounds for every cell of the kernel's box (nghost is at least 2), also
+// where that face is not computed.
+struct DonorIn {
+  double q[NHYDRO + 3], bx, dxw;
+};
+
+template <int DIR>
+__device__ __forceinline__ DonorIn donor_load(const MeshK &M, int g, int k, int j, int i,
+                                              const double *__restrict__ wb,
+                                              const double *__restrict__ bb, const FaceOut &o) {
+  const long s = (DIR == 0) ? 1 : ((DIR == 1) ? M.nc1 : static_cast<long>(M.nc1) * M.nc2);
+  const long c = cidx(M, k, j, i) - s;
+  DonorIn a;
+#pragma unroll
+  for (int n = 0; n < NHYDRO; ++n) a.q[n] = wb[n * M.ncell + c];
+#pragma unroll
+  for (int n = 0; n < 3; ++n)
+    if (n != IB1 + DIR) a.q[NHYDRO + n] = bb[n * M.ncell + c];
+  a.bx = o.bn[bidx<DIR>(M, g, k, j, i)];
+  a.dxw = ctab(M, g, DIR)[(DIR == 0) ? i : ((DIR == 1) ? j : k)];
+  return a;
+}
+
+template <int DIR, int RS, class FO>
+__device__ __forceinline__ void donor_face(const MeshK &M, int g, int k, int j, int i,
+                                           const DonorIn &a, const double *own,
+                                           const FO &o, double dt) {
+  constexpr int y = (DIR + 1) % 3, z = (DIR + 2) % 3;
+  constexpr int src[NWAVE] = {IDN, IVX + DIR, IVX + y, IVX + z, IPR, NHYDRO + y, NHYDRO + z};
+  double wl[NWAVE], wr[NWAVE], fx[NHYDRO];
+#pragma unroll
+  for (int v = 0; v < NWAVE; ++v) {
+    wl[v] = a.q[src[v]];
+    wr[v] = own[src[v]];
+  }
+  face_emit<DIR, RS>(M, g, k, j, i, wl, wr, a.bx, &a.dxw, o, dt, true, fx);
+  store_flux<DIR>(M, g, k, j, i, o, fx);
+}
+
+// Donor-cell launches load a face's inputs ahead of the face before, and the cell's own
+// values once for its three faces: at three wavefronts per SIMD the loads' latency was
+// exposed three times (VALU busy 63 %).  The 168 registers of that occupancy hold it (HLLD
+// with 6 spilled; the relativistic HLLD would spill dozens and keeps the other order).
+// 64 blocks of 64^3 cells, HLLD: 1.76 -> 1.49 ms; of 32^3: 252 -> 228 us.
+constexpr bool donor_ahead(int order, int rs) { return order == 1 && rs != 3; }
+constexpr int flux_min_waves(int order, int rs) { return donor_ahead(order, rs) ? 3 : 1; }
+
+// The unused first entry of a packed row: stored so that its cache line is whole.
+template <class FO>
+__device__ __forceinline__ void pad_row(const MeshK &M, int g, int k, int j, int i,
+                                        const FO &o) {
+  const long q = static_cast<long>(g) * M.fl[0].n + foidx<0>(M, k, j, i);
+  const double zero[NHYDRO] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  face_put(o, &o.ey[q], 0.0);
+  face_put(o, &o.ez[q], 0.0);
+  face_put(o, &o.wct[q], 0.0);
+  store_flux<0>(M, g, k, j, i, o, zero);
+}
+
 // One thread per cell of [is-1,ie+1]x[js-1,je+1]x[ks-1,ke+1]; each computes the faces on
 // its low sides that lie in the reference's loop ranges (calculate_fluxes.cpp:68-76,
 // 176-182, 299-302).
@@ -496,22 +565,34 @@ __device__ __forceinline__ void flux3_body(const MeshK &M, const double *__restr
   if (!map_kind(M, KK_FLUX, lw, nwg, T, g, i, j, k)) return;
   const double *wb = w + static_cast<long>(g) * NHYDRO * M.ncell;
   const double *bb = bcc + static_cast<long>(g) * 3 * M.ncell;
-  if (i >= M.is) {
-    flux_face<0, ORDER, RS>(M, g, k, j, i, wb, bb, o1, dt);
-  } else if (M.packed) {   // the row's unused first entry: complete its cache line
-    const long q = static_cast<long>(g) * M.fl[0].n + foidx<0>(M, k, j, i);
-    const double zero[NHYDRO] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    face_put(o1, &o1.ey[q], 0.0);
-    face_put(o1, &o1.ez[q], 0.0);
-    face_put(o1, &o1.wct[q], 0.0);
-    store_flux<0>(M, g, k, j, i, o1, zero);
+  if (donor_ahead(ORDER, RS)) {
+    double own[NHYDRO + 3];
+    const long c = cidx(M, k, j, i);
+    const DonorIn a1 = donor_load<0>(M, g, k, j, i, wb, bb, o1);
+#pragma unroll
+    for (int n = 0; n < NHYDRO; ++n) own[n] = wb[n * M.ncell + c];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) own[NHYDRO + n] = bb[n * M.ncell + c];
+    const DonorIn a2 = donor_load<1>(M, g, k, j, i, wb, bb, o2);
+    __builtin_amdgcn_sched_barrier(0);
+    if (i >= M.is) donor_face<0, RS>(M, g, k, j, i, a1, own, o1, dt);
+    else if (M.packed) pad_row(M, g, k, j, i, o1);
+    __builtin_amdgcn_sched_barrier(0);
+    const DonorIn a3 = donor_load<2>(M, g, k, j, i, wb, bb, o3);
+    __builtin_amdgcn_sched_barrier(0);
+    if (j >= M.js) donor_face<1, RS>(M, g, k, j, i, a2, own, o2, dt);
+    __builtin_amdgcn_sched_barrier(0);
+    if (k >= M.ks) donor_face<2, RS>(M, g, k, j, i, a3, own, o3, dt);
+    return;
   }
+  if (i >= M.is) flux_face<0, ORDER, RS>(M, g, k, j, i, wb, bb, o1, dt);
+  else if (M.packed) pad_row(M, g, k, j, i, o1);
   if (j >= M.js) flux_face<1, ORDER, RS>(M, g, k, j, i, wb, bb, o2, dt);
   if (k >= M.ks) flux_face<2, ORDER, RS>(M, g, k, j, i, wb, bb, o3, dt);
 }
 
 template <int ORDER, int RS, bool STREAM>
-__global__ void __launch_bounds__(WG) k_flux3(MeshK M, const double *__restrict__ w,
+__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS)) k_flux3(MeshK M, const double *__restrict__ w,
                                                const double *__restrict__ bcc, FaceOut o1,
                                                FaceOut o2, FaceOut o3,
                                                const Clock *__restrict__ clk, TileK T) {
@@ -1936,7 +2017,7 @@ __device__ __forceinline__ int2 ens_item(const int2 *__restrict__ map, int v) {
 }
 
 template <int ORDER, int RS, bool STREAM>
-__global__ void __launch_bounds__(WG) k_flux3_ens(const EnsMember *__restrict__ E,
+__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS)) k_flux3_ens(const EnsMember *__restrict__ E,
                                                    const int2 *__restrict__ map, int nwork) {
   for (int v = blockIdx.x; v < nwork; v += gridDim.x) {
     const int2 mw = ens_item(map, v);
@@ -2126,7 +2207,7 @@ __global__ void __launch_bounds__(WG) k_blk_riemann(MeshK M, int k, int j, int i
 
 // Hydro::CalculateFluxes on one block with dt by value (the fused three-direction body).
 template <int ORDER, int RS>
-__global__ void __launch_bounds__(WG) k_blk_flux3(MeshK M, const double *__restrict__ w,
+__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS)) k_blk_flux3(MeshK M, const double *__restrict__ w,
                                                   const double *__restrict__ bcc, FaceOut o1,
                                                   FaceOut o2, FaceOut o3, double dt) {
   flux3_body<ORDER, RS>(M, w, bcc, o1, o2, o3, dt, blockIdx.x, gridDim.x, TileK{0, 0, 0});
