@@ -65,10 +65,10 @@ class HipEvents:
 # linear), fetched KiB x 2.0 + written KiB x 1.0 (the factors a 512 MiB device copy
 # gives): profiles/vl2_hlld_plm_turbulence256_hbm_traffic.md.
 MEASURED_TRAFFIC = {
-    "flux_xyz_plm": 11396524816,
-    "flux_xyz_dc": 8299554176,
-    "update_u_b_ct": 7940971036,
-    "corner_emf": 3773546268,
+    "flux_xyz_plm": 10432512000,
+    "flux_xyz_dc": 7734272000,
+    "update_u_b_ct": 7601152000,
+    "corner_emf": 4796928000,
     "cons2prim": 3309664999,
     "ghost_exchange": 2299010489,
 }
@@ -79,7 +79,7 @@ MEASURED_FP64_FLOP = {
     "flux_xyz_plm": 47786607216,
     "flux_xyz_dc": 31422754608,
     "update_u_b_ct": 4173332480,
-    "corner_emf": 2422603776,
+    "corner_emf": 2592000000,
     "cons2prim": 3371907300,
 }
 FP64_PEAK = 78.6e12
