@@ -59,8 +59,9 @@ namespace {
 
 constexpr int WG = 256;
 
-// Layout of the per-face outputs along one direction (fluxes, face EMFs, CT weights) within
-// one block: element (k, j, i) at k * plane + j * row + i - org, n doubles per component.
+// Packed layout of a mesh's per-face outputs (fluxes, face EMFs, CT weights) within one block,
+// the same for the three directions (pack_faces): element (k, j, i) at
+// k * plane + j * row + i - org, n doubles per component.
 struct FaceLayout {
   int row, plane;
   long org, n;
@@ -75,8 +76,7 @@ struct MeshK {
   long ncell;                 // nc1*nc2*nc3
   long nf1, nf2, nf3;         // x1f, x2f, x3f face-array sizes per block
   long ne1, ne2, ne3;         // x1e, x2e, x3e edge-array sizes per block
-  FaceLayout fl[3];           // per-face outputs of direction d
-  int packed;                 // 1: packed layout, the same for the three (pack_faces)
+  FaceLayout fl;              // per-face outputs (packed; not used by the per-block entries)
   int cstride;                // doubles of coordinate table per block
   int coff[3];                // offset of direction d inside the table
   const int *nbr;             // [nblocks][27] same-level neighbour gid, -1 across an
@@ -115,10 +115,21 @@ __device__ __forceinline__ long f2idx(const MeshK &M, int k, int j, int i) {
 __device__ __forceinline__ long f3idx(const MeshK &M, int k, int j, int i) {
   return static_cast<long>(k) * (M.nc2 * M.nc1) + (j * M.nc1 + i);
 }
-template <int DIR>
+// Per-face outputs of direction DIR: packed on a mesh, in the extents of the face fields in
+// the arrays of a per-block caller.  The kind of layout is the kernel's: with both as run-time
+// strides (three of them in MeshK) the per-block fluxes spilled scalar registers and k_corner
+// over one block of 64^3 cells took 18.3 us in place of 15.6.
+template <int DIR, bool PACKED>
 __device__ __forceinline__ long foidx(const MeshK &M, int k, int j, int i) {
-  const FaceLayout &L = M.fl[DIR];
-  return static_cast<long>(k) * L.plane + (j * L.row + i) - L.org;
+  if (PACKED) return static_cast<long>(k) * M.fl.plane + (j * M.fl.row + i) - M.fl.org;
+  if (DIR == 0) return f1idx(M, k, j, i);
+  if (DIR == 1) return f2idx(M, k, j, i);
+  return f3idx(M, k, j, i);
+}
+template <int DIR, bool PACKED>
+__device__ __forceinline__ long fosize(const MeshK &M) {
+  if (PACKED) return M.fl.n;
+  return (DIR == 0) ? M.nf1 : ((DIR == 1) ? M.nf2 : M.nf3);
 }
 // edge arrays: x1e (nc3+1, nc2+1, nc1), x2e (nc3+1, nc2, nc1+1), x3e (nc3, nc2+1, nc1+1)
 __device__ __forceinline__ long e1idx(const MeshK &M, int k, int j, int i) {
@@ -309,6 +320,7 @@ __device__ __forceinline__ void ppm_cell(const double *q, double &qminus, double
 struct FaceOut {
   const double *bn;   // normal face field b.xNf
   double *flx, *ey, *ez, *wct;
+  static constexpr bool packed = true;
 };
 
 // The same registers stored streaming, past the L2 caches: for sets of outputs larger than
@@ -319,6 +331,11 @@ struct FaceOut {
 // the launch's, not chosen per store: a branch around each took PPM fluxes 659 -> 693 us.
 struct FaceOutStream : FaceOut {
   __device__ explicit FaceOutStream(const FaceOut &o) : FaceOut(o) {}
+};
+// The same registers in the arrays of a per-block caller.
+struct FaceOutBlock : FaceOut {
+  static constexpr bool packed = false;
+  __device__ explicit FaceOutBlock(const FaceOut &o) : FaceOut(o) {}
 };
 template <bool STREAM>
 using FaceOutOf = std::conditional_t<STREAM, FaceOutStream, FaceOut>;
@@ -425,7 +442,8 @@ __device__ __forceinline__ void face_emit(const MeshK &M, int g, int k, int j, i
   fx[ivz] = f[IVZ];
   fx[IEN] = f[IEN];
   if (emit) {
-    const long q = static_cast<long>(g) * M.fl[DIR].n + foidx<DIR>(M, k, j, i);
+    const long q = static_cast<long>(g) * fosize<DIR, FO::packed>(M) +
+                   foidx<DIR, FO::packed>(M, k, j, i);
     face_put(o, &o.ey[q], -f[IBY]);
     face_put(o, &o.ez[q], f[IBZ]);
     face_put(o, &o.wct[q], ct_weight(f[IDN], wl[IDN], wr[IDN], *dxw, dt));
@@ -454,8 +472,8 @@ __device__ __forceinline__ void face_solve(const MeshK &M, int g, int k, int j, 
 template <int DIR, class FO>
 __device__ __forceinline__ void store_flux(const MeshK &M, int g, int k, int j, int i,
                                            const FO &o, const double *fx) {
-  const long nf = M.fl[DIR].n;
-  double *fb = o.flx + static_cast<long>(g) * NHYDRO * nf + foidx<DIR>(M, k, j, i);
+  const long nf = fosize<DIR, FO::packed>(M);
+  double *fb = o.flx + static_cast<long>(g) * NHYDRO * nf + foidx<DIR, FO::packed>(M, k, j, i);
 #pragma unroll
   for (int n = 0; n < NHYDRO; ++n) face_put(o, &fb[n * nf], fx[n]);
 }
@@ -536,16 +554,22 @@ __device__ __forceinline__ void donor_face(const MeshK &M, int g, int k, int j, 
 // Donor-cell launches load a face's inputs ahead of the face before, and the cell's own
 // values once for its three faces: at three wavefronts per SIMD the loads' latency was
 // exposed three times (VALU busy 63 %).  The 168 registers of that occupancy hold it (HLLD
-// with 6 spilled; the relativistic HLLD would spill dozens and keeps the other order).
-// 64 blocks of 64^3 cells, HLLD: 1.76 -> 1.49 ms; of 32^3: 252 -> 228 us.
-constexpr bool donor_ahead(int order, int rs) { return order == 1 && rs != 3; }
-constexpr int flux_min_waves(int order, int rs) { return donor_ahead(order, rs) ? 3 : 1; }
+// with 4 spilled; the relativistic HLLD would spill dozens and keeps the other order).
+// 256^3 cells in blocks of 32^3, HLLD: 1.76 -> 1.49 ms; 128^3: 252 -> 228 us.  HLLD in the
+// layout of a per-block caller spills 10 and keeps the other order too (100x80x80 cells: 69.8
+// us ahead, 66.8 not, 48^3 17.3 and 16.8; HLLE over 96x80x80 54.4 ahead, 57.1 not).
+constexpr bool donor_ahead(int order, int rs, bool packed) {
+  return order == 1 && rs != 3 && (packed || rs != 0);
+}
+constexpr int flux_min_waves(int order, int rs, bool packed) {
+  return donor_ahead(order, rs, packed) ? 3 : 1;
+}
 
 // The unused first entry of a packed row: stored so that its cache line is whole.
 template <class FO>
 __device__ __forceinline__ void pad_row(const MeshK &M, int g, int k, int j, int i,
                                         const FO &o) {
-  const long q = static_cast<long>(g) * M.fl[0].n + foidx<0>(M, k, j, i);
+  const long q = static_cast<long>(g) * M.fl.n + foidx<0, true>(M, k, j, i);
   const double zero[NHYDRO] = {0.0, 0.0, 0.0, 0.0, 0.0};
   face_put(o, &o.ey[q], 0.0);
   face_put(o, &o.ez[q], 0.0);
@@ -565,7 +589,7 @@ __device__ __forceinline__ void flux3_body(const MeshK &M, const double *__restr
   if (!map_kind(M, KK_FLUX, lw, nwg, T, g, i, j, k)) return;
   const double *wb = w + static_cast<long>(g) * NHYDRO * M.ncell;
   const double *bb = bcc + static_cast<long>(g) * 3 * M.ncell;
-  if (donor_ahead(ORDER, RS)) {
+  if (donor_ahead(ORDER, RS, FO::packed)) {
     double own[NHYDRO + 3];
     const long c = cidx(M, k, j, i);
     const DonorIn a1 = donor_load<0>(M, g, k, j, i, wb, bb, o1);
@@ -576,7 +600,7 @@ __device__ __forceinline__ void flux3_body(const MeshK &M, const double *__restr
     const DonorIn a2 = donor_load<1>(M, g, k, j, i, wb, bb, o2);
     __builtin_amdgcn_sched_barrier(0);
     if (i >= M.is) donor_face<0, RS>(M, g, k, j, i, a1, own, o1, dt);
-    else if (M.packed) pad_row(M, g, k, j, i, o1);
+    else if (FO::packed) pad_row(M, g, k, j, i, o1);
     __builtin_amdgcn_sched_barrier(0);
     const DonorIn a3 = donor_load<2>(M, g, k, j, i, wb, bb, o3);
     __builtin_amdgcn_sched_barrier(0);
@@ -586,16 +610,15 @@ __device__ __forceinline__ void flux3_body(const MeshK &M, const double *__restr
     return;
   }
   if (i >= M.is) flux_face<0, ORDER, RS>(M, g, k, j, i, wb, bb, o1, dt);
-  else if (M.packed) pad_row(M, g, k, j, i, o1);
+  else if (FO::packed) pad_row(M, g, k, j, i, o1);
   if (j >= M.js) flux_face<1, ORDER, RS>(M, g, k, j, i, wb, bb, o2, dt);
   if (k >= M.ks) flux_face<2, ORDER, RS>(M, g, k, j, i, wb, bb, o3, dt);
 }
 
 template <int ORDER, int RS, bool STREAM>
-__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS)) k_flux3(MeshK M, const double *__restrict__ w,
-                                               const double *__restrict__ bcc, FaceOut o1,
-                                               FaceOut o2, FaceOut o3,
-                                               const Clock *__restrict__ clk, TileK T) {
+__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS, true))
+    k_flux3(MeshK M, const double *__restrict__ w, const double *__restrict__ bcc, FaceOut o1,
+            FaceOut o2, FaceOut o3, const Clock *__restrict__ clk, TileK T) {
   using FO = FaceOutOf<STREAM>;
   flux3_body<ORDER, RS>(M, w, bcc, FO(o1), FO(o2), FO(o3), clk->dt,
                         xcd_logical_wg(M.xcd_remap & XCD_FLUX), gridDim.x, T);
@@ -1008,7 +1031,7 @@ __device__ __forceinline__ void corner_edges(int k, int j, int i, FW1 W1F, FW2 W
   }
 }
 
-template <bool SR>
+template <bool SR, bool PACKED>
 __device__ __forceinline__ void corner_body(const MeshK &M, const CornerArgs &ca, int lw,
                                             int nwg, TileK T) {
   int g, i, j, k;
@@ -1017,22 +1040,23 @@ __device__ __forceinline__ void corner_body(const MeshK &M, const CornerArgs &ca
   const double *__restrict__ bcc = ca.bcc;
   const double *wb = w + static_cast<long>(g) * NHYDRO * M.ncell;
   const double *bb = bcc + static_cast<long>(g) * 3 * M.ncell;
-  const long o1 = g * M.fl[0].n, o2 = g * M.fl[1].n, o3 = g * M.fl[2].n;
+  const long o1 = g * fosize<0, PACKED>(M), o2 = g * fosize<1, PACKED>(M);
+  const long o3 = g * fosize<2, PACKED>(M);
   const double *__restrict__ wx1 = ca.wx1 + o1, *__restrict__ wx2 = ca.wx2 + o2;
   const double *__restrict__ wx3 = ca.wx3 + o3;
   const double *__restrict__ e2x1 = ca.e2x1 + o1, *__restrict__ e3x1 = ca.e3x1 + o1;
   const double *__restrict__ e1x2 = ca.e1x2 + o2, *__restrict__ e3x2 = ca.e3x2 + o2;
   const double *__restrict__ e1x3 = ca.e1x3 + o3, *__restrict__ e2x3 = ca.e2x3 + o3;
   double *__restrict__ e1 = ca.e1, *__restrict__ e2 = ca.e2, *__restrict__ e3 = ca.e3;
-  auto W1F = [&](int kk, int jj, int ii) { return wx1[foidx<0>(M, kk, jj, ii)]; };
-  auto W2F = [&](int kk, int jj, int ii) { return wx2[foidx<1>(M, kk, jj, ii)]; };
-  auto W3F = [&](int kk, int jj, int ii) { return wx3[foidx<2>(M, kk, jj, ii)]; };
-  auto E2X1 = [&](int kk, int jj, int ii) { return e2x1[foidx<0>(M, kk, jj, ii)]; };
-  auto E3X1 = [&](int kk, int jj, int ii) { return e3x1[foidx<0>(M, kk, jj, ii)]; };
-  auto E1X2 = [&](int kk, int jj, int ii) { return e1x2[foidx<1>(M, kk, jj, ii)]; };
-  auto E3X2 = [&](int kk, int jj, int ii) { return e3x2[foidx<1>(M, kk, jj, ii)]; };
-  auto E1X3 = [&](int kk, int jj, int ii) { return e1x3[foidx<2>(M, kk, jj, ii)]; };
-  auto E2X3 = [&](int kk, int jj, int ii) { return e2x3[foidx<2>(M, kk, jj, ii)]; };
+  auto W1F = [&](int kk, int jj, int ii) { return wx1[foidx<0, PACKED>(M, kk, jj, ii)]; };
+  auto W2F = [&](int kk, int jj, int ii) { return wx2[foidx<1, PACKED>(M, kk, jj, ii)]; };
+  auto W3F = [&](int kk, int jj, int ii) { return wx3[foidx<2, PACKED>(M, kk, jj, ii)]; };
+  auto E2X1 = [&](int kk, int jj, int ii) { return e2x1[foidx<0, PACKED>(M, kk, jj, ii)]; };
+  auto E3X1 = [&](int kk, int jj, int ii) { return e3x1[foidx<0, PACKED>(M, kk, jj, ii)]; };
+  auto E1X2 = [&](int kk, int jj, int ii) { return e1x2[foidx<1, PACKED>(M, kk, jj, ii)]; };
+  auto E3X2 = [&](int kk, int jj, int ii) { return e3x2[foidx<1, PACKED>(M, kk, jj, ii)]; };
+  auto E1X3 = [&](int kk, int jj, int ii) { return e1x3[foidx<2, PACKED>(M, kk, jj, ii)]; };
+  auto E2X3 = [&](int kk, int jj, int ii) { return e2x3[foidx<2, PACKED>(M, kk, jj, ii)]; };
   auto cc = [&](int comp, int kk, int jj, int ii) {
     return cc_e<SR>(M, wb, bb, comp, cidx(M, kk, jj, ii));
   };
@@ -1094,25 +1118,22 @@ struct MarchPlane {
 };
 
 __device__ __forceinline__ MarchPlane march_load(const MeshK &M, const CornerArgs &ca, int g,
-                                                 int k, unsigned oc, unsigned o1, unsigned o2) {
-  asm volatile("" : "+v"(oc), "+v"(o1), "+v"(o2));
+                                                 int k, unsigned oc, unsigned of) {
+  asm volatile("" : "+v"(oc), "+v"(of));
   const long n = M.ncell, pc = static_cast<long>(M.nc2) * M.nc1;
-  // rows of x2 and x3 faces have the same pitch in either layout
-  const long q1 = g * M.fl[0].n + static_cast<long>(k) * M.fl[0].plane - M.fl[0].org;
-  const long q2 = g * M.fl[1].n + static_cast<long>(k) * M.fl[1].plane - M.fl[1].org;
-  const long q3 = g * M.fl[2].n + static_cast<long>(k) * M.fl[2].plane - M.fl[2].org;
+  const long q = g * M.fl.n + static_cast<long>(k) * M.fl.plane - M.fl.org;
   const double *w = ca.w + static_cast<long>(g) * NHYDRO * n + k * pc;
   const double *b = ca.bcc + static_cast<long>(g) * 3 * n + k * pc;
   MarchPlane P;
-  P.w1 = ldb(ca.wx1 + q1, o1);
-  P.e2x1 = ldb(ca.e2x1 + q1, o1);
-  P.e3x1 = ldb(ca.e3x1 + q1, o1);
-  P.w2 = ldb(ca.wx2 + q2, o2);
-  P.e1x2 = ldb(ca.e1x2 + q2, o2);
-  P.e3x2 = ldb(ca.e3x2 + q2, o2);
-  P.w3 = ldb(ca.wx3 + q3, o2);
-  P.e1x3 = ldb(ca.e1x3 + q3, o2);
-  P.e2x3 = ldb(ca.e2x3 + q3, o2);
+  P.w1 = ldb(ca.wx1 + q, of);
+  P.e2x1 = ldb(ca.e2x1 + q, of);
+  P.e3x1 = ldb(ca.e3x1 + q, of);
+  P.w2 = ldb(ca.wx2 + q, of);
+  P.e1x2 = ldb(ca.e1x2 + q, of);
+  P.e3x2 = ldb(ca.e3x2 + q, of);
+  P.w3 = ldb(ca.wx3 + q, of);
+  P.e1x3 = ldb(ca.e1x3 + q, of);
+  P.e2x3 = ldb(ca.e2x3 + q, of);
   P.vx = ldb(w + IVX * n, oc);
   P.vy = ldb(w + IVY * n, oc);
   P.vz = ldb(w + IVZ * n, oc);
@@ -1144,11 +1165,10 @@ __device__ __forceinline__ void corner_march(const MeshK &M, const CornerArgs &c
   const bool live = t < ncs && i <= iend && j <= jend;
   const bool act = live && ri > 0 && rj > 0;
   const unsigned oc = 8u * static_cast<unsigned>(j * M.nc1 + i);
-  const unsigned o1 = 8u * static_cast<unsigned>(j * M.fl[0].row + i);
-  const unsigned o2 = 8u * static_cast<unsigned>(j * M.fl[1].row + i);
+  const unsigned of = 8u * static_cast<unsigned>(j * M.fl.row + i);
   const unsigned oe = 8u * static_cast<unsigned>(j * (M.nc1 + 1) + i);
   MarchPlane C{}, N{};
-  if (live) C = march_load(M, ca, g, k0 - 1, oc, o1, o2);
+  if (live) C = march_load(M, ca, g, k0 - 1, oc, of);
   // plane k-1: own face values, cell-centred E1 of this cell and one row down, E2 of this
   // cell and one column left
   double w1p = 0.0, w2p = 0.0, e12p = 0.0, e21p = 0.0, c0p = 0.0, c0jp = 0.0, c1p = 0.0;
@@ -1176,7 +1196,7 @@ __device__ __forceinline__ void corner_march(const MeshK &M, const CornerArgs &c
       S[7 * ncs + t] = cc0;
       S[8 * ncs + t] = cc1;
       S[9 * ncs + t] = cc2;
-      if (k + 1 < k1) N = march_load(M, ca, g, k + 1, oc, o1, o2);
+      if (k + 1 < k1) N = march_load(M, ca, g, k + 1, oc, of);
     }
     __syncthreads();
     if (act) {
@@ -1232,9 +1252,9 @@ __device__ __forceinline__ void corner_march(const MeshK &M, const CornerArgs &c
   }
 }
 
-template <bool SR>
+template <bool SR, bool PACKED>
 __global__ void __launch_bounds__(WG) k_corner(MeshK M, CornerArgs ca, TileK T) {
-  corner_body<SR>(M, ca, xcd_logical_wg(M.xcd_remap & XCD_CORNER), gridDim.x, T);
+  corner_body<SR, PACKED>(M, ca, xcd_logical_wg(M.xcd_remap & XCD_CORNER), gridDim.x, T);
 }
 
 template <bool SR>
@@ -1365,14 +1385,14 @@ __device__ __forceinline__ void update_cell_u(const MeshK &M, int g, int k, int 
   const double vol = dx1[i] * dx2[j] * dx3[k];
   const long c = cidx(M, k, j, i);
   const long b0 = static_cast<long>(g) * NHYDRO * M.ncell;
-  const FaceLayout &L2 = M.fl[PACKED ? 0 : 1], &L3 = M.fl[PACKED ? 0 : 2];
-  const long n1 = M.fl[0].n, n2 = L2.n, n3 = L3.n;
+  const long n1 = fosize<0, PACKED>(M), n2 = fosize<1, PACKED>(M), n3 = fosize<2, PACKED>(M);
   const double *F1 = f1 + static_cast<long>(g) * NHYDRO * n1;
   const double *F2 = f2 + static_cast<long>(g) * NHYDRO * n2;
   const double *F3 = f3 + static_cast<long>(g) * NHYDRO * n3;
-  const long x1 = foidx<0>(M, k, j, i), x2 = foidx<PACKED ? 0 : 1>(M, k, j, i);
-  const long x3 = foidx<PACKED ? 0 : 2>(M, k, j, i);
-  const long sx2 = L2.row, sx3 = L3.plane;
+  const long x1 = foidx<0, PACKED>(M, k, j, i), x2 = foidx<1, PACKED>(M, k, j, i);
+  const long x3 = foidx<2, PACKED>(M, k, j, i);
+  const long sx2 = PACKED ? M.fl.row : M.nc1;
+  const long sx3 = PACKED ? M.fl.plane : static_cast<long>(M.nc2) * M.nc1;
 #pragma unroll
   for (int n = 0; n < NHYDRO; ++n) {
     double dflx = (a1 * F1[n * n1 + x1 + 1] - a1 * F1[n * n1 + x1]);
@@ -2017,8 +2037,8 @@ __device__ __forceinline__ int2 ens_item(const int2 *__restrict__ map, int v) {
 }
 
 template <int ORDER, int RS, bool STREAM>
-__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS)) k_flux3_ens(const EnsMember *__restrict__ E,
-                                                   const int2 *__restrict__ map, int nwork) {
+__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS, true))
+    k_flux3_ens(const EnsMember *__restrict__ E, const int2 *__restrict__ map, int nwork) {
   for (int v = blockIdx.x; v < nwork; v += gridDim.x) {
     const int2 mw = ens_item(map, v);
     const EnsMember &e = E[mw.x];
@@ -2034,7 +2054,7 @@ __global__ void __launch_bounds__(WG) k_corner_ens(const EnsMember *__restrict__
   for (int v = blockIdx.x; v < nwork; v += gridDim.x) {
     const int2 mw = ens_item(map, v);
     const EnsMember &e = E[mw.x];
-    corner_body<SR>(e.M, e.ca, mw.y, e.nwg[1], e.tile[1]);
+    corner_body<SR, true>(e.M, e.ca, mw.y, e.nwg[1], e.tile[1]);
   }
 }
 
@@ -2207,10 +2227,12 @@ __global__ void __launch_bounds__(WG) k_blk_riemann(MeshK M, int k, int j, int i
 
 // Hydro::CalculateFluxes on one block with dt by value (the fused three-direction body).
 template <int ORDER, int RS>
-__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS)) k_blk_flux3(MeshK M, const double *__restrict__ w,
-                                                  const double *__restrict__ bcc, FaceOut o1,
-                                                  FaceOut o2, FaceOut o3, double dt) {
-  flux3_body<ORDER, RS>(M, w, bcc, o1, o2, o3, dt, blockIdx.x, gridDim.x, TileK{0, 0, 0});
+__global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS, false))
+    k_blk_flux3(MeshK M, const double *__restrict__ w, const double *__restrict__ bcc,
+                FaceOut o1, FaceOut o2, FaceOut o3, double dt) {
+  using FO = FaceOutBlock;
+  flux3_body<ORDER, RS>(M, w, bcc, FO(o1), FO(o2), FO(o3), dt, blockIdx.x, gridDim.x,
+                        TileK{0, 0, 0});
 }
 
 // Field::CT (what & 2) and Hydro::AddFluxDivergence (what & 1) of one block, in place on
@@ -2380,11 +2402,9 @@ __device__ __forceinline__ refops::View face_view(const MeshK &M, double *p, int
   const long nf = (c == 0) ? M.nf1 : ((c == 1) ? M.nf2 : M.nf3);
   return refops::View{p + static_cast<long>(g) * nf, M.nc2 + (c == 1), M.nc1 + (c == 0)};
 }
-__device__ __forceinline__ refops::View flux_view(const MeshK &M, double *p, int g, int n,
-                                                  int c) {
-  const FaceLayout L = (c == 0) ? M.fl[0] : ((c == 1) ? M.fl[1] : M.fl[2]);
-  return refops::View{p + (static_cast<long>(g) * NHYDRO + n) * L.n - L.org, L.plane / L.row,
-                      L.row};
+__device__ __forceinline__ refops::View flux_view(const MeshK &M, double *p, int g, int n) {
+  return refops::View{p + (static_cast<long>(g) * NHYDRO + n) * M.fl.n - M.fl.org,
+                      M.fl.plane / M.fl.row, M.fl.row};
 }
 __device__ __forceinline__ refops::View edge_view(const MeshK &M, const double *p, int g,
                                                   int c) {
@@ -2461,7 +2481,7 @@ __device__ __forceinline__ void smr_bcc_p2c(const MeshK &M, const SmrArgs &a, in
 // (k, j, i) (LoadFluxBoundaryBufferToCoarser, flux_correction_cc.cpp:77-166).
 __device__ __forceinline__ double smr_flux_restrict(const MeshK &M, const SmrArgs &a, int dir,
                                                     int src, int n, int k, int j, int i) {
-  const refops::View f = flux_view(M, a.flux[dir], src, n, dir);
+  const refops::View f = flux_view(M, a.flux[dir], src, n);
   const double *d1 = ctab(M, src, 0), *d2 = ctab(M, src, 1), *d3 = ctab(M, src, 2);
   if (dir == 0) {
     const double amm = d2[j] * d3[k], amp = d2[j + 1] * d3[k];
@@ -2564,7 +2584,7 @@ __global__ void __launch_bounds__(smrplan::CHUNK_THREADS) k_smr(MeshK M, SmrArgs
           smr_bcc_p2c(M, a, g, k, j, i);
           break;
         case smrplan::FLUX_RESTRICT: {
-          const refops::View f = flux_view(M, a.flux[c], g, n, c);
+          const refops::View f = flux_view(M, a.flux[c], g, n);
           f(k, j, i) = smr_flux_restrict(M, a, c, st.src, n, sk, sj, si);
           break;
         }
@@ -2769,39 +2789,24 @@ bool tile_ok(int kind, int t) { return TILES[t].tx >= 0 || kind == KK_CORNER; }
 // A single mesh also runs the flux kernel's z-march (k_flux_zm); ensembles do not.
 bool mesh_tile_ok(int kind, int t) { return tile_ok(kind, t) || kind == KK_FLUX; }
 
-// Layouts of the per-face outputs.  public: the extents of the face fields, as a MeshBlock
-// holds them (the per-block entries).  packed: all three directions over the flux kernel's
-// box [is-1,ie+1] x [js-1,je+1] x [ks-1,ke+1] and nothing else, each component padded to
-// whole cache lines, so that a work-group's 256 consecutive cells write whole lines.  With
-// the unused ends of each row in between, nearly every second line is written in part, and
-// such lines take HBM 1.5 to 1.8 times as long: the 24 arrays alone of 64 blocks of 32^3
-// cells 265 against 153 us (a kernel that only copies).  DC fluxes over 64 blocks of 64^3
-// cells 1.99 -> 1.76 ms, corner EMFs 0.70 -> 0.66 (64 of 32^3: 120 -> 106 us; a refined mesh
-// of 16^3 blocks: 91 -> 69); the update 1.20 -> 1.23 ms.
-void public_faces(MeshK &M) {
-  const long nf[3] = {M.nf1, M.nf2, M.nf3};
-  for (int d = 0; d < 3; ++d) {
-    M.fl[d].row = M.nc1 + (d == 0);
-    M.fl[d].plane = M.fl[d].row * (M.nc2 + (d == 1));
-    M.fl[d].org = 0;
-    M.fl[d].n = nf[d];
-  }
-  M.packed = 0;
-}
-
+// Per-face outputs over the flux kernel's box [is-1,ie+1] x [js-1,je+1] x [ks-1,ke+1] and
+// nothing else, each component padded to whole cache lines, so that a work-group's 256
+// consecutive cells write whole lines.  In the extents of the face fields, with the unused ends
+// of each row in between, nearly every second line is written in part, and such lines take HBM
+// 1.5 to 1.8 times as long: the 24 arrays alone of 64 blocks of 32^3 cells 265 against 153 us
+// (a kernel that only copies).  Over 256^3 cells in blocks of 32^3, DC fluxes 1.99 -> 1.76 ms,
+// corner EMFs 0.70 -> 0.66 (128^3: 120 -> 106 us; a refined mesh of 16^3 blocks: 91 -> 69); the
+// update 1.20 -> 1.23 ms.
 void pack_faces(MeshK &M) {
-  for (int d = 0; d < 3; ++d) {
-    M.fl[d].row = M.nx1 + 2;
-    M.fl[d].plane = (M.nx1 + 2) * (M.nx2 + 2);
-    M.fl[d].org = static_cast<long>(M.ks - 1) * M.fl[d].plane +
-                  static_cast<long>(M.js - 1) * M.fl[d].row + (M.is - 1);
-    M.fl[d].n = (static_cast<long>(M.fl[d].plane) * (M.nx3 + 2) + 15) / 16 * 16;
-  }
-  M.packed = 1;
+  M.fl.row = M.nx1 + 2;
+  M.fl.plane = (M.nx1 + 2) * (M.nx2 + 2);
+  M.fl.org = static_cast<long>(M.ks - 1) * M.fl.plane +
+             static_cast<long>(M.js - 1) * M.fl.row + (M.is - 1);
+  M.fl.n = (static_cast<long>(M.fl.plane) * (M.nx3 + 2) + 15) / 16 * 16;
 }
 
 // Bytes of a mesh's packed per-face outputs: eight for each of the three faces of a cell.
-double face_bytes(const MeshK &M) { return 24.0 * sizeof(double) * M.fl[0].n * M.nblocks; }
+double face_bytes(const MeshK &M) { return 24.0 * sizeof(double) * M.fl.n * M.nblocks; }
 
 // Whether a flux launch that writes this much streams it: more than the 4 MB of L2 in each
 // of the 8 XCDs.
@@ -2818,14 +2823,14 @@ int face_register(int what, int *ncomp) {
 // Moves the faces that the flux kernel computes along d between one block's public array
 // and its packed one.
 void copy_faces(const MeshK &M, int d, int ncomp, double *pub, double *packed, bool pack) {
-  MeshK P = M;
-  public_faces(P);
-  const FaceLayout &A = P.fl[d], &B = M.fl[d];
+  const FaceLayout &B = M.fl;
+  const long nf[3] = {M.nf1, M.nf2, M.nf3};
+  const long row = M.nc1 + (d == 0), plane = row * (M.nc2 + (d == 1));
   for (int n = 0; n < ncomp; ++n)
     for (int k = M.ks - (d != 2); k <= M.ke + 1; ++k)
       for (int j = M.js - (d != 1); j <= M.je + 1; ++j) {
         const int i0 = M.is - (d != 0);
-        double *a = pub + n * A.n + static_cast<long>(k) * A.plane + j * A.row + i0;
+        double *a = pub + n * nf[d] + k * plane + j * row + i0;
         double *b = packed + n * B.n + static_cast<long>(k) * B.plane + j * B.row + i0 - B.org;
         const size_t bytes = sizeof(double) * (M.ie + 2 - i0);
         if (pack) std::memcpy(b, a, bytes);
@@ -3020,9 +3025,9 @@ int launch_corner_args(ath_mesh *m, const CornerArgs &ca) {
   else if (T.tx < 0)
     hipLaunchKernelGGL((k_corner_march<false>), grid, dim3(WG), lds, m->stream, M, ca, T);
   else if (m->d.relativistic)
-    hipLaunchKernelGGL((k_corner<true>), grid, dim3(WG), 0, m->stream, M, ca, T);
+    hipLaunchKernelGGL((k_corner<true, true>), grid, dim3(WG), 0, m->stream, M, ca, T);
   else
-    hipLaunchKernelGGL((k_corner<false>), grid, dim3(WG), 0, m->stream, M, ca, T);
+    hipLaunchKernelGGL((k_corner<false, true>), grid, dim3(WG), 0, m->stream, M, ca, T);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -3902,16 +3907,16 @@ int mesh_build(const ath_mesh_desc *desc, const std::vector<smrplan::BlockInfo> 
   for (int q = 0; q < 3 && !rc; ++q) {
     rc |= m->alloc(&m->b[q], nf[q] * nb);
     rc |= m->alloc(&m->bb[q], nf[q] * nb);
-    rc |= m->alloc(&m->flux[q], NHYDRO * M.fl[q].n * nb);
-    rc |= m->alloc(&m->wx[q], M.fl[q].n * nb);
+    rc |= m->alloc(&m->flux[q], NHYDRO * M.fl.n * nb);
+    rc |= m->alloc(&m->wx[q], M.fl.n * nb);
   }
   if (!rc) {
-    rc |= m->alloc(&m->e2x1, M.fl[0].n * nb);
-    rc |= m->alloc(&m->e3x1, M.fl[0].n * nb);
-    rc |= m->alloc(&m->e1x2, M.fl[1].n * nb);
-    rc |= m->alloc(&m->e3x2, M.fl[1].n * nb);
-    rc |= m->alloc(&m->e1x3, M.fl[2].n * nb);
-    rc |= m->alloc(&m->e2x3, M.fl[2].n * nb);
+    rc |= m->alloc(&m->e2x1, M.fl.n * nb);
+    rc |= m->alloc(&m->e3x1, M.fl.n * nb);
+    rc |= m->alloc(&m->e1x2, M.fl.n * nb);
+    rc |= m->alloc(&m->e3x2, M.fl.n * nb);
+    rc |= m->alloc(&m->e1x3, M.fl.n * nb);
+    rc |= m->alloc(&m->e2x3, M.fl.n * nb);
     rc |= m->alloc(&m->e[0], M.ne1 * nb);
     rc |= m->alloc(&m->e[1], M.ne2 * nb);
     rc |= m->alloc(&m->e[2], M.ne3 * nb);
@@ -4071,7 +4076,7 @@ int ath_gpu_set_block(ath_mesh_t m, int gid, int what, const double *host) {
   const int d = face_register(what, &nc);
   if (d >= 0) try {
     // the computed faces to the packed array; the others are kept for ath_gpu_get_block
-    const long np = nc * m->M.fl[d].n;
+    const long np = nc * m->M.fl.n;
     std::vector<double> packed(np, 0.0), rest(host, host + n);
     copy_faces(m->M, d, nc, rest.data(), packed.data(), true);
     {
@@ -4100,7 +4105,7 @@ int ath_gpu_get_block(ath_mesh_t m, int gid, int what, double *host) {
   int nc;
   const int d = face_register(what, &nc);
   if (d >= 0) try {
-    const long np = nc * m->M.fl[d].n;
+    const long np = nc * m->M.fl.n;
     std::vector<double> packed(np);
     HIPCHK(hipMemcpyAsync(packed.data(), *pool + gid * np, sizeof(double) * np,
                           hipMemcpyDeviceToHost, m->stream));
@@ -4843,7 +4848,6 @@ int ath_gpu_block_create(const ath_block_desc *d, ath_block_t *out) {
   M.ne1 = static_cast<long>(M.nc3 + 1) * (M.nc2 + 1) * M.nc1;
   M.ne2 = static_cast<long>(M.nc3 + 1) * M.nc2 * (M.nc1 + 1);
   M.ne3 = static_cast<long>(M.nc3) * (M.nc2 + 1) * (M.nc1 + 1);
-  public_faces(M);
   M.coff[0] = 0;
   M.coff[1] = 3 * M.nc1;
   M.coff[2] = 3 * (M.nc1 + M.nc2);
@@ -5015,8 +5019,8 @@ int ath_gpu_block_compute_corner_e(ath_block_t b, const double *w, const double 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const TileK T{0, 0, 0};
   const dim3 g(static_cast<unsigned>(kind_chunks(M, KK_CORNER, T)));
-  if (b->relativistic) hipLaunchKernelGGL((k_corner<true>), g, dim3(WG), 0, st, M, ca, T);
-  else hipLaunchKernelGGL((k_corner<false>), g, dim3(WG), 0, st, M, ca, T);
+  if (b->relativistic) hipLaunchKernelGGL((k_corner<true, false>), g, dim3(WG), 0, st, M, ca, T);
+  else hipLaunchKernelGGL((k_corner<false, false>), g, dim3(WG), 0, st, M, ca, T);
   return blk_check_stream(st);
 }
 

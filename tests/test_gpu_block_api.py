@@ -16,6 +16,7 @@ import pytest
 
 from athena_amd.gpu import AthGpuError, Block
 from athena_amd.mesh import MeshDesc
+from athena_amd.pgen.blast import Blast
 from athena_amd.pgen.sr import ShearLayer
 from athena_amd.pgen.turbulence import Turbulence, turbulence_mesh
 from oracle_bind import OracleMesh
@@ -98,6 +99,25 @@ def test_calculate_fluxes_corner_ct_divergence(case):
         for n in ("b1", "b2", "b3", "u"):
             same(d.get(n), o.get(0, n), "order %d %s" % (order, n))
     blk.close()
+
+
+@pytest.mark.parametrize("nx,sr,rsolver,ng", [((5, 9, 7), False, "hlld", 3),
+                                              ((8, 3, 13), False, "hlle", 3),
+                                              ((2, 2, 2), False, "hlld", 2),
+                                              ((6, 11, 4), True, "hlle", 3),
+                                              ((4, 7, 10), True, "hlld", 3)])
+def test_stage_on_uneven_edges(nx, sr, rsolver, ng):
+    """Three different extents, so that a row or plane stride of another direction or of a
+    mesh's packed per-face arrays would show."""
+    print("case block api, uneven edges", nx, sr, rsolver, flush=True)
+    m = MeshDesc(nx=nx, bnx=nx, xmin=(-0.5,) * 3, xmax=(0.5,) * 3, cfl=0.3, xorder=2, ng=ng,
+                 gamma=4.0 / 3.0 if sr else 5.0 / 3.0, rsolver=rsolver, relativistic=sr)
+    ic = (ShearLayer if sr else Blast)(m)
+    o = OracleMesh(m)
+    o.load([ic.block(0)])
+    o.initialize()
+    o.run(2)
+    test_calculate_fluxes_corner_ct_divergence((m, o))
 
 
 def test_cons2prim_ranges_and_new_dt(case):
