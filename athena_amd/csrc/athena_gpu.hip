@@ -117,8 +117,8 @@ __device__ __forceinline__ long f3idx(const MeshK &M, int k, int j, int i) {
 }
 // Per-face outputs of direction DIR: packed on a mesh, in the extents of the face fields in
 // the arrays of a per-block caller.  The kind of layout is the kernel's: with both as run-time
-// strides (three of them in MeshK) the per-block fluxes spilled scalar registers and k_corner
-// over one block of 64^3 cells took 18.3 us in place of 15.6.
+// strides (three of them in MeshK) the per-block fluxes spilled scalar registers, and one stage
+// over a block of 64^3 cells took 118.8 us against 118.2.
 template <int DIR, bool PACKED>
 __device__ __forceinline__ long foidx(const MeshK &M, int k, int j, int i) {
   if (PACKED) return static_cast<long>(k) * M.fl.plane + (j * M.fl.row + i) - M.fl.org;
@@ -628,7 +628,8 @@ __global__ void __launch_bounds__(WG, flux_min_waves(ORDER, RS, true))
 // qp[v] for the seven face-state variables in the rotated order of DIR.  The interface at
 // index fc along DIR takes wl = qp of cell fc-1 and wr = qm of cell fc, the same
 // expressions face_flux evaluates (PLM: pf and mf of plm.cpp:149-155; PPM: ppm_cell).
-template <int DIR, int ORDER>
+// OPAQUE keeps the PPM limiters' selects out of the solver's own branches (as in face_flux).
+template <int DIR, int ORDER, bool OPAQUE>
 __device__ __forceinline__ void recon_cell(const MeshK &M, int g, int k, int j, int i,
                                            const double *__restrict__ wb,
                                            const double *__restrict__ bb, double *qm,
@@ -665,6 +666,10 @@ __device__ __forceinline__ void recon_cell(const MeshK &M, int g, int k, int j, 
 #pragma unroll
       for (int m = 0; m < 5; ++m) q[m] = src[c + (m - 2) * s];
       ppm_cell(q, qm[v], qp[v]);
+      if (OPAQUE) {
+        asm volatile("" : "+v"(qm[v]), "+v"(qp[v]));
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
 }
@@ -723,7 +728,10 @@ __host__ __device__ __forceinline__ bool fzm_pos(const MeshK &M, const FzmGeom &
 // the face are reconstructed by the lane, as in k_flux3.  Every state is the value
 // face_flux computes for that face, so the fluxes, EMFs and weights are the same bits.
 // Not bounded to k_flux3's 3 wavefronts per SIMD: at 168 VGPRs the spills cost more
-// (PLM launch 3.40 against 2.84 ms at 256^3) than the third wavefront gains.
+// (PLM launch 3.40 against 2.84 ms at 256^3) than the third wavefront gains.  The
+// relativistic HLLD takes PPM states opaque: folded into its branches they need 276 registers,
+// one wavefront per SIMD, and the launch over 128^3 1931 us against 1614 (208 registers); the
+// other solvers are faster with them folded in (HLLD 710 us, opaque 736).
 template <int ORDER, int RS>
 __global__ void __launch_bounds__(WG) k_flux_zm(MeshK M, const double *__restrict__ w,
                                                  const double *__restrict__ bcc, FaceOut o1,
@@ -737,11 +745,12 @@ __global__ void __launch_bounds__(WG) k_flux_zm(MeshK M, const double *__restric
   const bool in = fzm_pos(M, G, wv, lane, g0, j0, i0, k0, k1);
   const bool own = in && lane > 0;
   const double dt = clk->dt;
+  constexpr bool OPAQUE = RS == 3;
 
   double p3[NWAVE] = {};   // high-face x3 states of cell (k-1, j, i)
   if (k0 >= M.ks) {
     double m3[NWAVE];
-    recon_cell<2, ORDER>(M, g0, k0 - 1, j0, i0, w + static_cast<long>(g0) * NHYDRO * M.ncell,
+    recon_cell<2, ORDER, OPAQUE>(M, g0, k0 - 1, j0, i0, w + static_cast<long>(g0) * NHYDRO * M.ncell,
                          bcc + static_cast<long>(g0) * 3 * M.ncell, m3, p3);
   }
 #pragma unroll 1
@@ -757,12 +766,14 @@ __global__ void __launch_bounds__(WG) k_flux_zm(MeshK M, const double *__restric
     const double *bb = bcc + static_cast<long>(g) * 3 * M.ncell;
     double wl[NWAVE], wr[NWAVE], fx[NHYDRO];
     // x1: this lane's cell, left states from the lane before
-    recon_cell<0, ORDER>(M, g, k, j, i, wb, bb, wr, wl);
+    recon_cell<0, ORDER, OPAQUE>(M, g, k, j, i, wb, bb, wr, wl);
 #pragma unroll
     for (int v = 0; v < NWAVE; ++v) wl[v] = __shfl_up(wl[v], 1, 64);
     if (live && i >= M.is) {
       face_solve<0, ORDER, RS>(M, g, k, j, i, wl, wr, o1, dt, true, fx);
       store_flux<0>(M, g, k, j, i, o1, fx);
+    } else if (live) {
+      pad_row(M, g, k, j, i, o1);
     }
     // x2: both cells (indices made opaque again, so that the x1 addresses are not kept
     // alive through the x1 solve for reuse here)
@@ -771,8 +782,8 @@ __global__ void __launch_bounds__(WG) k_flux_zm(MeshK M, const double *__restric
     bb = bcc + static_cast<long>(g) * 3 * M.ncell;
     if (live && j >= M.js) {
       double t[NWAVE];
-      recon_cell<1, ORDER>(M, g, k, j - 1, i, wb, bb, t, wl);
-      recon_cell<1, ORDER>(M, g, k, j, i, wb, bb, wr, t);
+      recon_cell<1, ORDER, OPAQUE>(M, g, k, j - 1, i, wb, bb, t, wl);
+      recon_cell<1, ORDER, OPAQUE>(M, g, k, j, i, wb, bb, wr, t);
       face_solve<1, ORDER, RS>(M, g, k, j, i, wl, wr, o2, dt, true, fx);
       store_flux<1>(M, g, k, j, i, o2, fx);
     }
@@ -780,7 +791,7 @@ __global__ void __launch_bounds__(WG) k_flux_zm(MeshK M, const double *__restric
     asm volatile("" : "+v"(k), "+v"(g), "+v"(j), "+v"(i));
     wb = w + static_cast<long>(g) * NHYDRO * M.ncell;
     bb = bcc + static_cast<long>(g) * 3 * M.ncell;
-    recon_cell<2, ORDER>(M, g, k, j, i, wb, bb, wr, wl);
+    recon_cell<2, ORDER, OPAQUE>(M, g, k, j, i, wb, bb, wr, wl);
     if (live && k >= M.ks) {
       face_solve<2, ORDER, RS>(M, g, k, j, i, p3, wr, o3, dt, true, fx);
       store_flux<2>(M, g, k, j, i, o3, fx);

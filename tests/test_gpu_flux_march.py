@@ -33,9 +33,10 @@ def _turb(n, bn, **kw):
     return m, Turbulence(m)
 
 
-def _sr_hlld():
+def _sr_hlld(xorder=2):
     m = MeshDesc(nx=(32, 32, 32), bnx=(16, 16, 16), xmin=(-0.5,) * 3, xmax=(0.5,) * 3,
-                 gamma=4.0 / 3.0, cfl=0.3, xorder=2, ng=2, rsolver="hlld", relativistic=True)
+                 gamma=4.0 / 3.0, cfl=0.3, xorder=xorder, ng=xorder, rsolver="hlld",
+                 relativistic=True)
     return m, ShearLayer(m)
 
 
@@ -64,7 +65,8 @@ CASES = {
     "turb_dc_hlle": lambda: _turb(32, 16, rsolver="hlle", xorder=1),
     "turb_ppm_hlld_outflow": lambda: _turb(16, 8, xorder=3, ng=3, bc=OUTFLOW),
     "sr_shear_ppm_hlle": _sr_ppm,
-    "sr_shear_plm_hlld": _sr_hlld,
+    "sr_shear_ppm_hlld": lambda: _sr_hlld(3),
+    "sr_shear_plm_hlld": lambda: _sr_hlld(2),
     "smr_linwave_plm_hlld": _smr,
 }
 
