@@ -1091,8 +1091,9 @@ __device__ __forceinline__ void corner_body(const MeshK &M, const CornerArgs &ca
 // Bound by the vector caches (their lines wait on L2 for 80 % of the launch) and by the
 // partly written lines at the row ends (10 % in a bare copy of the same pattern).  Every
 // value loaded per edge that needs it, between two barriers a plane, in segments of 8
-// planes, took 132 us over 64 blocks of 32^3 cells, 772 us over 64 of 64^3, 27 us over 64
-// of 16^3; each loaded once, 118, 698 and 17 us.
+// planes, took 131 us over 64 blocks of 32^3 cells, 773 us over 512 of them, 29 us over 64
+// of 16^3 and 26 us over one of 32x16x16; each loaded once, from packed faces and in
+// segments of corner_tile's height, 82, 611, 19 and 7 us.
 struct MarchGeom {
   int ti, tj, nti, ntj, ks, nks;
 };
@@ -2653,7 +2654,7 @@ struct ath_mesh {
   double *dtpart = nullptr;
   long ndtpart = 0;           // capacity of dtpart
   long ndt_used = 0;          // entries written by the last cons2prim with dt
-  // per work kind: linear chunks, the corner kernel's z-march over 8 planes
+  // per work kind: linear chunks, the corner kernel's z-march (TILES[6])
   TileK tile[4] = {{0, 0, 0}, {-1, 0, 8}, {0, 0, 0}, {0, 0, 0}};
   int fdiv_rows = 0;          // > 0: stages use k_flux_div with bands of this many rows
   // ath_gpu_cycle as one captured HIP graph per cycle (ath_gpu_mesh_set_graph)
@@ -2790,8 +2791,8 @@ long kind_chunks(const MeshK &M, int kind, TileK T) {
 }
 
 // Tile shapes the autotuner chooses from (index 0: linear chunks); indices 6 and 7 are
-// the z-march: the corner kernel's (k_corner_march, segments of at most 2 and 4 planes) and,
-// on single meshes, the flux kernel's (k_flux_zm, segments of 8 and 16 planes).
+// the z-march: the corner kernel's (k_corner_march, segment heights of corner_tile) and, on
+// single meshes, the flux kernel's (k_flux_zm, segments of 8 and 16 planes).
 constexpr int NTILES = 8;
 constexpr TileK TILES[NTILES] = {{0, 0, 0}, {64, 4, 1}, {32, 8, 1}, {16, 16, 1}, {16, 4, 4},
                                  {8, 8, 4}, {-1, 0, 8}, {-1, 0, 16}};
@@ -2849,18 +2850,26 @@ void copy_faces(const MeshK &M, int d, int ncomp, double *pub, double *packed, b
       }
 }
 
-// The z-march tile of a corner launch: segments of 2 planes (tile option 6) or 4 (7), one
-// where that would leave the GPU's 256 CUs short of three work-groups each.  Low segments
-// reload a plane more often but sweep memory nearly in order: segments of 1, 2, 3, 4, 8 and
-// 33 planes take 809, 699, 754, 755, 782 and 831 us over 64 blocks of 64^3 cells, 122, 118,
-// 122, 121, 123 and 122 us over 64 of 32^3.  One mesh of 8 blocks of 16^3: 7.0 us with
-// single planes, 8.3 with two.  share: this mesh's part of the launch (1 by itself).
+// The z-march tile of a corner launch.  A segment loads one plane, and a tile one row of
+// cells, more than it writes; low segments sweep memory nearly in order.  So a tile of few rows
+// (wide MeshBlocks) takes tall segments, a tile of many rows low ones: 16 planes over the tile's
+// rows, at least 2 (tile option 6), and half as many again (option 7).  us in segments of
+// 2 / 3 / 4 / 8 / 16 planes, the rule's height of option 6 in brackets:
+//   512 blocks of 32^3    636 [611] 639  694  718     64 of 32^3    87  [81] 80   80   83
+//    64 blocks of 64^3    709  673  646 [610] 608      8 of 64^3    93   90  87  [84]  85
+//     8 blocks of 96^3    368  357  338  310 [303]     8 of 128^3  785  726 709  647 [629]
+//    64 blocks of 40^3    161 [151] 148  154  161      8 of 48^3    40   39 [38]  35   37
+//   512 blocks of 16^3   [101] 102  100  100  103
+// The height falls where it would leave the GPU's 256 CUs short of three work-groups each: 8
+// blocks of 16^3 take 7.8 us in single planes, 7.6 in two, 8.8 in three; one of 32x16x16 6.8,
+// 7.7 and 8.6.  share: this mesh's part of the launch (1 by itself).
 TileK corner_tile(const MeshK &M, TileK T, double share) {
   if (T.tx >= 0) return T;
   const MarchGeom G = march_geom(M, T.tz);
   const double planes = static_cast<double>(G.nti) * G.ntj * (M.nx3 + 1) * M.nblocks;
   const int h = static_cast<int>(planes / (3.0 * 256.0 * share) + 0.5);
-  T.tz = std::max(1, std::min(T.tz / 4, h));
+  const int tall = std::max(2, (32 / G.tj + 1) / 2);   // 16 over the rows, rounded
+  T.tz = std::max(1, std::min((T.tz == 8) ? tall : tall + tall / 2, h));
   return T;
 }
 

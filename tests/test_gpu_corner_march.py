@@ -1,8 +1,9 @@
 """GPU checks of the corner EMF kernel's z-march (tile options 6, the default, and 7) where
 its tiles and segments have edges: rows of edges that fill a work-group, that just fit and
 that are split into equal tiles; the smallest MeshBlocks; MeshBlocks whose planes do not
-divide into whole segments; and launches tall enough for segments of two and four planes as
-well as single ones.  The march evaluates the linear mapping's expressions on the same
+divide into whole segments; and launches of every kind of height: single planes, the two
+planes at least of a large launch, and the tallest segments, of tiles of one and of several
+rows, with the height each case reaches checked against the launch's rule.  The march evaluates the linear mapping's expressions on the same
 values, so whole runs are bit for bit those of one thread per edge (tile 0), which the
 parity tests tie to the CPU oracle; the widest case is compared with the oracle directly."""
 import numpy as np
@@ -32,15 +33,35 @@ def _lw(bnx):
     return m, LinearWave(m, wave_flag=0, amp=1e-6)
 
 
+# name: mesh, planes per segment under tile options 6 and 7
 CASES = {
-    "2x2x2": lambda: _lw((2, 2, 2)),
-    "3x4x6": lambda: _lw((3, 4, 6)),
-    "row_126": lambda: _box((126, 6, 5), (126, 6, 5)),     # 127 edges: one tile, 128 cells
-    "row_127": lambda: _box((127, 6, 5), (127, 6, 5)),     # 128 edges: two tiles
-    "row_260_sr": lambda: _box((260, 4, 7), (260, 4, 7), sr=True),   # three tiles
-    "segments_of_4": lambda: _box((70, 70, 66), (35, 35, 33)),
-    "segments_of_4_sr": lambda: _box((60, 60, 60), (20, 20, 20), sr=True),
+    "2x2x2": (lambda: _lw((2, 2, 2)), 2, 2),
+    "3x4x6": (lambda: _lw((3, 4, 6)), 1, 1),
+    "row_126": (lambda: _box((126, 6, 5), (126, 6, 5)), 1, 1),   # 127 edges: one tile, 128 cells
+    "row_127": (lambda: _box((127, 6, 5), (127, 6, 5)), 1, 1),   # 128 edges: two tiles
+    "row_260_sr": (lambda: _box((260, 4, 7), (260, 4, 7), sr=True), 1, 1),   # three tiles
+    "rows_of_5": (lambda: _box((70, 140, 66), (35, 35, 33)), 3, 4),
+    "rows_of_1": (lambda: _box((192, 96, 64), (96, 48, 32)), 11, 17),   # 33 planes in 3 and 2
+    "rows_of_7_sr": (lambda: _box((80, 60, 60), (20, 20, 20), sr=True), 2, 3),
 }
+
+
+def heights(m):
+    """Planes per segment under tile options 6 and 7 (corner_tile and march_geom)."""
+    n = [b + 1 for b in m.bnx]
+    ti = n[0] if n[0] < 256 else 255
+    if ti > 127:
+        ti = -(-n[0] // -(-n[0] // 127))
+    nti, tj = -(-n[0] // ti), 256 // (ti + 1) - 1
+    ntj = -(-n[1] // tj)
+    tj = -(-n[1] // ntj)
+    tall = max(2, (32 // tj + 1) // 2)
+    short = int(nti * ntj * n[2] * m.nblocks / 768.0 + 0.5)
+    out = []
+    for cap in (tall, tall + tall // 2):
+        h = max(1, min(cap, short))
+        out.append(-(-n[2] // -(-n[2] // h)))
+    return tuple(out)
 
 
 def run(m, ic, tiles):
@@ -54,8 +75,10 @@ def run(m, ic, tiles):
 
 @pytest.mark.parametrize("name", list(CASES))
 def test_corner_march_runs_bit_for_bit_as_one_thread_per_edge(name):
-    m, ic = CASES[name]()
+    make, *want = CASES[name]
+    m, ic = make()
     print("case corner march", name, flush=True)
+    assert heights(m) == tuple(want)
     ref = run(m, ic, [0, 0, 0, 0])
     for tile in (6, 7):
         d = run(m, ic, [0, tile, 0, 0])

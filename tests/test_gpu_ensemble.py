@@ -182,7 +182,7 @@ def test_single_mesh_tiles_and_autotune(solo):
     d2.run(4)
     assert_same(snapshot(d2), snaps[3][2])
     for tiles in ([0, 6, 0, 0], [0, 7, 0, 0]):
-        # the corner kernel's z-march, 8 and 16 planes per segment
+        # the corner kernel's z-march, both segment heights
         d3 = fresh([(m, ic)])[0]
         d3.set_tiles(tiles)
         assert list(d3.tiles()) == tiles
