@@ -323,12 +323,10 @@ struct FaceOut {
   static constexpr bool packed = true;
 };
 
-// The same registers stored streaming, past the L2 caches: for sets of outputs larger than
-// those, which the next kernels read from memory either way, so that the rows a launch's
-// stencils share stay cached.  At 256^3 (64 blocks of 64^3 cells) PLM fluxes 2.36 -> 2.27 ms,
-// DC 1.76 -> 1.63, corner EMFs 0.66 -> 0.64; 128^3 (32^3) corner EMFs 106 -> 90 us; a mesh
-// of 32^3 cells (9 MB of outputs), streamed: update 15.2 -> 16.9 us.  The kind of store is
-// the launch's, not chosen per store: a branch around each took PPM fluxes 659 -> 693 us.
+// The same registers stored streaming, past the L2 caches: for sets of outputs that the
+// kernels reading them take from memory either way (stream_faces), so that the rows a launch's
+// stencils share stay cached.  The kind of store is the launch's, not chosen per store: a
+// branch around each took PPM fluxes 659 -> 693 us.
 struct FaceOutStream : FaceOut {
   __device__ explicit FaceOutStream(const FaceOut &o) : FaceOut(o) {}
 };
@@ -2820,9 +2818,16 @@ void pack_faces(MeshK &M) {
 // Bytes of a mesh's packed per-face outputs: eight for each of the three faces of a cell.
 double face_bytes(const MeshK &M) { return 24.0 * sizeof(double) * M.fl.n * M.nblocks; }
 
-// Whether a flux launch that writes this much streams it: more than the 4 MB of L2 in each
-// of the 8 XCDs.
-bool stream_faces(double bytes) { return bytes > 32.0 * (1 << 20); }
+// Whether a flux launch that writes this much streams it: more than about half of the 256 MB
+// cache in front of HBM, whose other half then holds what the next kernels read besides.  Flux,
+// corner and update launches of one cycle together, us with ordinary stores / streaming:
+//    53 MB (one 64^3)   161/164     58 (8 of 32^3)  173/172    68 (64 of 16^3)   191/193
+//    86 (12 of 32^3)    230/236    102 (126x64x64)  252/258   109 (8 of 40^3)    273/273
+//   115 (16 of 32^3)    283/284    130 (18 of 32^3) 313/308   143 (8 of 44^3)    346/331
+//   154 (8 of 48x48x40) 373/360    172 (one 96^3)   452/428   183 (8 of 48^3)    429/406
+//   231 (216 of 16^3)   581/536    461 (64 of 32^3) 1066/998
+// (PLM HLLD; 183 HLLE).  PPM: 58 MB 224/225, 109 353/356, 143 462/453.
+bool stream_faces(double bytes) { return bytes > 120.0 * (1 << 20); }
 
 // The per-face output register `what` as (direction, components), or direction -1.
 int face_register(int what, int *ncomp) {

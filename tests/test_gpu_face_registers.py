@@ -7,7 +7,9 @@ import pytest
 from athena_amd.gpu import Ensemble, GpuMesh
 from athena_amd.mesh import MeshDesc
 from athena_amd.pgen.blast import Blast
+from athena_amd.pgen.sr import ShearLayer
 from oracle_bind import OracleMesh
+from test_gpu_smr import compare, load_both, smr_wave
 
 pytestmark = pytest.mark.gpu
 REGS = ("flux1", "flux2", "flux3", "wght1", "wght2", "wght3")
@@ -62,16 +64,30 @@ def test_face_registers(nx, bnx, ng):
         assert np.array_equal(got[rest], a[rest]), (g, reg)
 
 
-@pytest.mark.parametrize("bnx,nx,rsolver,xorder", [((16, 16, 16), (48, 48, 64), "hlld", 2),
-                                                   ((27, 16, 29), (54, 64, 58), "hlle", 3)])
-def test_streamed_faces(bnx, nx, rsolver, xorder):
-    """More than 32 MB of per-face outputs: the flux launches store them past the L2 caches.
-    A mesh by itself and, with a smaller one, in an ensemble."""
-    m = MeshDesc(nx=nx, bnx=bnx, xmin=(-0.5,) * 3, xmax=(0.5,) * 3, gamma=5.0 / 3.0, cfl=0.3,
-                 xorder=xorder, ng=xorder if xorder == 2 else 4, rsolver=rsolver)
-    print("case streamed faces", nx, bnx, rsolver, flush=True)
-    assert 24 * 8 * m.nblocks * np.prod([n + 2 for n in bnx]) > 32 * 2**20
-    blocks = [Blast(m).block(g) for g in range(m.nblocks)]
+STREAMED = 120 * 2**20   # bytes of per-face outputs above which a launch stores them streaming
+
+
+def face_bytes(m):
+    return 24 * 8 * m.nblocks * np.prod([n + 2 for n in m.bnx])
+
+
+@pytest.mark.parametrize("bnx,nx,sr,rsolver,xorder",
+                         [((24, 24, 24), (96, 96, 72), False, "hlld", 2),
+                          ((27, 16, 29), (81, 96, 87), False, "hlle", 3),
+                          ((25, 24, 23), (100, 72, 92), True, "hlle", 3),
+                          ((24, 24, 24), (96, 96, 72), True, "hlld", 2)])
+def test_streamed_faces(bnx, nx, sr, rsolver, xorder):
+    """Enough per-face outputs that the flux launches store them past the L2 caches.  A mesh by
+    itself and, with a smaller one, in an ensemble."""
+    ng = xorder if xorder == 2 else 4
+    desc = dict(xmin=(-0.5,) * 3, xmax=(0.5,) * 3, gamma=4.0 / 3.0 if sr else 5.0 / 3.0, cfl=0.3,
+                xorder=xorder, ng=ng, rsolver=rsolver, relativistic=sr)
+    ic = ShearLayer if sr else Blast
+    m = MeshDesc(nx=nx, bnx=bnx, **desc)
+    print("case streamed faces", nx, bnx, sr, rsolver, flush=True)
+    assert face_bytes(m) > STREAMED
+    problem = ic(m)
+    blocks = [problem.block(g) for g in range(m.nblocks)]
     o = OracleMesh(m)
     o.load(blocks)
     o.initialize(1e300)
@@ -81,10 +97,9 @@ def test_streamed_faces(bnx, nx, rsolver, xorder):
         d.load(blocks)
         d.initialize(1e300)
     dev[0].run(2)
-    small = MeshDesc(nx=bnx, bnx=bnx, xmin=(-0.5,) * 3, xmax=(0.5,) * 3, gamma=5.0 / 3.0,
-                     cfl=0.3, xorder=xorder, ng=m.ng, rsolver=rsolver)
+    small = MeshDesc(nx=bnx, bnx=bnx, **desc)
     s = GpuMesh(small)
-    s.load([Blast(small).block(0)])
+    s.load([ic(small).block(0)])
     s.initialize(1e300)
     e = Ensemble([dev[1], s])
     e.run(2)
@@ -92,3 +107,16 @@ def test_streamed_faces(bnx, nx, rsolver, xorder):
         for g in range(m.nblocks):
             for key in ("u", "b1", "b2", "b3"):
                 assert np.array_equal(d.get(g, key).ravel(), o.get(g, key).ravel()), (g, key)
+
+
+def test_streamed_faces_of_a_refined_mesh():
+    """The flux and EMF corrections read and write what the streamed launch stored."""
+    m, lw = smr_wave(80, 0, xorder=2, rsolver="hlld", ng=2)
+    print("case streamed faces, refined", m.nblocks, flush=True)
+    assert face_bytes(m) > STREAMED
+    dev, ora = load_both(m, lw)
+    dev.initialize(1.0)
+    ora.initialize(1.0)
+    dev.run(2, 1.0)
+    ora.run(2, 1.0)
+    compare(dev, ora, m, "after 2 cycles")
