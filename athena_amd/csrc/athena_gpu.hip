@@ -2688,7 +2688,8 @@ struct ath_mesh {
   double prof_ms[64] = {0};
   long prof_cnt[64] = {0};
 
-  // entries of per-face registers outside the packed arrays, as the caller last set them
+  // entries of per-face registers outside the packed arrays, as the caller last set them, in
+  // the order of the public array (walk_faces); none where all are zero
   std::map<std::pair<int, int>, std::vector<double>> unpacked;
   std::mutex unpacked_mutex;
 
@@ -2837,21 +2838,26 @@ int face_register(int what, int *ncomp) {
   return -1;
 }
 
-// Moves the faces that the flux kernel computes along d between one block's public array
-// and its packed one.
-void copy_faces(const MeshK &M, int d, int ncomp, double *pub, double *packed, bool pack) {
+// Walks one block's public array of a per-face register in order: inside(public offset, packed
+// offset, count) for the faces that the flux kernel computes along d, outside(public offset,
+// count) for the rest.
+template <class In, class Out>
+void walk_faces(const MeshK &M, int d, int ncomp, In inside, Out outside) {
   const FaceLayout &B = M.fl;
-  const long nf[3] = {M.nf1, M.nf2, M.nf3};
-  const long row = M.nc1 + (d == 0), plane = row * (M.nc2 + (d == 1));
+  const long ext[3] = {M.nc1 + (d == 0), M.nc2 + (d == 1), M.nc3 + (d == 2)};
+  const int i0 = M.is - (d != 0), i1 = M.ie + 2;
   for (int n = 0; n < ncomp; ++n)
-    for (int k = M.ks - (d != 2); k <= M.ke + 1; ++k)
-      for (int j = M.js - (d != 1); j <= M.je + 1; ++j) {
-        const int i0 = M.is - (d != 0);
-        double *a = pub + n * nf[d] + k * plane + j * row + i0;
-        double *b = packed + n * B.n + static_cast<long>(k) * B.plane + j * B.row + i0 - B.org;
-        const size_t bytes = sizeof(double) * (M.ie + 2 - i0);
-        if (pack) std::memcpy(b, a, bytes);
-        else std::memcpy(a, b, bytes);
+    for (int k = 0; k < ext[2]; ++k)
+      for (int j = 0; j < ext[1]; ++j) {
+        const long row = ((n * ext[2] + k) * ext[1] + j) * ext[0];
+        if (k < M.ks - (d != 2) || k > M.ke + 1 || j < M.js - (d != 1) || j > M.je + 1) {
+          outside(row, ext[0]);
+          continue;
+        }
+        outside(row, static_cast<long>(i0));
+        inside(row + i0, n * B.n + static_cast<long>(k) * B.plane + j * B.row + i0 - B.org,
+               static_cast<long>(i1 - i0));
+        outside(row + i1, ext[0] - i1);
       }
 }
 
@@ -4100,17 +4106,31 @@ int ath_gpu_set_block(ath_mesh_t m, int gid, int what, const double *host) {
   int nc;
   const int d = face_register(what, &nc);
   if (d >= 0) try {
-    // the computed faces to the packed array; the others are kept for ath_gpu_get_block
+    // the computed faces to the packed array; the others, unless all are zero, are kept for
+    // ath_gpu_get_block
     const long np = nc * m->M.fl.n;
-    std::vector<double> packed(np, 0.0), rest(host, host + n);
-    copy_faces(m->M, d, nc, rest.data(), packed.data(), true);
-    {
-      const std::lock_guard<std::mutex> lock(m->unpacked_mutex);
-      m->unpacked[{what, gid}] = std::move(rest);
+    std::vector<double> packed(np, 0.0), rest;
+    bool zero = true;
+    const double none[1] = {0.0};
+    long nrest = 0;
+    walk_faces(m->M, d, nc,
+               [&](long a, long b, long c) { std::copy(host + a, host + a + c, &packed[b]); },
+               [&](long a, long c) {
+                 nrest += c;
+                 for (long q = a; zero && q < a + c; ++q)
+                   zero = std::memcmp(host + q, none, sizeof(double)) == 0;
+               });
+    if (!zero) {
+      rest.reserve(nrest);
+      walk_faces(m->M, d, nc, [](long, long, long) {},
+                 [&](long a, long c) { rest.insert(rest.end(), host + a, host + a + c); });
     }
     HIPCHK(hipMemcpyAsync(*pool + gid * np, packed.data(), sizeof(double) * np,
                           hipMemcpyHostToDevice, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
+    const std::lock_guard<std::mutex> lock(m->unpacked_mutex);
+    if (zero) m->unpacked.erase({what, gid});
+    else m->unpacked[{what, gid}] = std::move(rest);
     return 0;
   } catch (const std::exception &e) {
     return fail(e.what());
@@ -4135,13 +4155,19 @@ int ath_gpu_get_block(ath_mesh_t m, int gid, int what, double *host) {
     HIPCHK(hipMemcpyAsync(packed.data(), *pool + gid * np, sizeof(double) * np,
                           hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
-    {
-      const std::lock_guard<std::mutex> lock(m->unpacked_mutex);
-      const auto rest = m->unpacked.find({what, gid});
-      if (rest != m->unpacked.end()) std::copy(rest->second.begin(), rest->second.end(), host);
-      else std::fill(host, host + n, 0.0);
-    }
-    copy_faces(m->M, d, nc, host, packed.data(), false);
+    const std::lock_guard<std::mutex> lock(m->unpacked_mutex);
+    const auto kept = m->unpacked.find({what, gid});
+    const double *rest = (kept != m->unpacked.end()) ? kept->second.data() : nullptr;
+    walk_faces(m->M, d, nc,
+               [&](long a, long b, long c) { std::copy_n(&packed[b], c, host + a); },
+               [&](long a, long c) {
+                 if (!rest) {
+                   std::fill_n(host + a, c, 0.0);
+                 } else {
+                   std::copy_n(rest, c, host + a);
+                   rest += c;
+                 }
+               });
     return 0;
   } catch (const std::exception &e) {
     return fail(e.what());

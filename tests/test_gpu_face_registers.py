@@ -1,6 +1,8 @@
 """GPU checks of the per-face registers (fluxes and CT weights), which a mesh keeps packed
 over the computed faces only: what a caller sets comes back whole, the computed faces hold
 the oracle's values in the array extents the caller sees, and the rest stays as set."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -62,6 +64,55 @@ def test_face_registers(nx, bnx, ng):
         rest = np.ones(a.shape, bool)
         rest[(...,) + comp] = False
         assert np.array_equal(got[rest], a[rest]), (g, reg)
+
+
+class _Mallinfo2(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_size_t) for n in ("arena", "ordblks", "smblks", "hblks", "hblkhd",
+                                               "usmblks", "fsmblks", "uordblks", "fordblks",
+                                               "keepcost")]
+
+
+def _host_bytes():
+    """Bytes the process holds from malloc."""
+    f = ctypes.CDLL(None).mallinfo2
+    f.restype = _Mallinfo2
+    s = f()
+    return s.uordblks + s.hblkhd
+
+
+def test_host_memory_of_set_registers():
+    """Setting the flux registers keeps on the host what lies outside the packed arrays, and
+    nothing where that is zero."""
+    m, _ = _mesh((96, 96, 96), (48, 48, 48), 2)
+    print("case host memory of face registers", flush=True)
+    d = GpuMesh(m)
+    n = m.bnx
+    regs = ("flux1", "flux2", "flux3")
+    full, zeroed, outside = {}, {}, 0
+    rng = np.random.default_rng(3)
+    for reg in regs:
+        x = int(reg[-1]) - 1
+        full[reg] = rng.standard_normal(_shape(m, reg))
+        zeroed[reg] = np.zeros_like(full[reg])
+        comp = tuple(slice(m.ng - (q != x), m.ng + n[q] + 1) for q in (2, 1, 0))
+        zeroed[reg][(...,) + comp] = full[reg][(...,) + comp]
+        outside += full[reg].nbytes - full[reg][(...,) + comp].nbytes
+    for arrays, keep in ((zeroed, 0), (full, outside * m.nblocks), (zeroed, 0)):
+        for reg in regs:       # staging buffers and the like
+            d.set(0, reg, zeroed[reg])
+            d.get(0, reg)
+        before = _host_bytes()
+        for g in range(m.nblocks):
+            for reg in regs:
+                d.set(g, reg, arrays[reg])
+        grown = _host_bytes() - before
+        assert grown < keep + 2**20, (grown, keep)
+        for g in (0, m.nblocks - 1):
+            for reg in regs:
+                assert np.array_equal(d.get(g, reg).ravel(), arrays[reg].ravel()), (g, reg)
+    minus = np.full(_shape(m, "wght1"), -0.0)
+    d.set(1, "wght1", minus)
+    assert np.signbit(d.get(1, "wght1")).all()
 
 
 STREAMED = 120 * 2**20   # bytes of per-face outputs above which a launch stores them streaming
