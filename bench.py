@@ -24,8 +24,8 @@ sys.path.insert(0, ROOT)
 import numpy as np  # noqa: E402
 
 HBM_PEAK = 8.0e12          # MI355X HBM3E, B/s
-TILE_NAMES = ("linear", "64x4x1", "32x8x1", "16x16x1", "16x4x4", "8x8x4", "zmarch8",
-              "zmarch16")
+TILE_NAMES = ("linear", "64x4x1", "32x8x1", "16x16x1", "16x4x4", "8x8x4", "zmarch_low",
+              "zmarch_high")
 BYTES_PER_ZONE_CYCLE = 536  # compulsory FP64 traffic of one VL2 MHD zone-cycle
 METRIC = "zone-cycles/s on 1 MI355X (3D MHD VL2+PLM+HLLD FP64) + % peak HBM GB/s"
 
@@ -60,27 +60,27 @@ class HipEvents:
         return ms.value
 
 
-# HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE on the
-# default workload (256^3 as 512 MeshBlocks of 32^3; tiles linear, zmarch8, linear,
+# Bytes per launch between L2 and memory measured with rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE on the
+# default workload (256^3 as 512 MeshBlocks of 32^3; tiles linear, zmarch_low, linear,
 # linear), fetched KiB x 2.0 + written KiB x 1.0 (the factors a 512 MiB device copy
 # gives): profiles/vl2_hlld_plm_turbulence256_hbm_traffic.md.
 MEASURED_TRAFFIC = {
-    "flux_xyz_plm": 10432512000,
-    "flux_xyz_dc": 7734272000,
-    "update_u_b_ct": 7601152000,
-    "corner_emf": 4796928000,
-    "cons2prim": 3309664999,
-    "ghost_exchange": 2299010489,
+    "flux_xyz_plm": 10419701760,
+    "flux_xyz_dc": 7732425933,
+    "update_u_b_ct": 7603234509,
+    "corner_emf": 4361470054,
+    "cons2prim": 3309685760,
+    "ghost_exchange": 2299034010,
 }
-TRAFFIC_TILES = ["linear", "zmarch8", "linear", "linear"]
+TRAFFIC_TILES = ["linear", "zmarch_low", "linear", "linear"]
 # FP64 FLOP per launch (64 x (ADD + MUL + 2 FMA) of the SQ_INSTS_VALU_*_F64 counters) on
 # the same workload: profiles/vl2_hlld_plm_turbulence256_fp64_valu.md.
 MEASURED_FP64_FLOP = {
-    "flux_xyz_plm": 47786607216,
-    "flux_xyz_dc": 31422754608,
+    "flux_xyz_plm": 47786607206,
+    "flux_xyz_dc": 31296771264,
     "update_u_b_ct": 4173332480,
-    "corner_emf": 2592000000,
-    "cons2prim": 3371907300,
+    "corner_emf": 2549809152,
+    "cons2prim": 3371907296,
 }
 FP64_PEAK = 78.6e12
 TRAFFIC_SOURCE = "profiles/vl2_hlld_plm_turbulence256_hbm_traffic.md"
@@ -735,9 +735,9 @@ def main():
                  "achieved": zcs * BYTES_PER_ZONE_CYCLE / 1e9, "unit": "GB/s",
                  "frac": zcs * BYTES_PER_ZONE_CYCLE / HBM_PEAK}
     if measured and all(k in MEASURED_TRAFFIC for k in stats if k != "new_dt"):
-        # the HBM bytes the cycle's launches actually move (the profile's counters times
-        # this run's launches per cycle) over this run's cycle time: how busy HBM is,
-        # beside the compulsory 536-byte figure above
+        # the bytes the cycle's launches exchange between L2 and memory (the profile's
+        # counters times this run's launches per cycle) over this run's cycle time, beside
+        # the compulsory 536-byte figure above; the 256 MB cache before HBM serves a part
         per_cycle = sum(MEASURED_TRAFFIC[k] * c / args.steps for k, (_, c) in stats.items()
                         if k != "new_dt")
         step_roof["measured_traffic"] = {
